@@ -192,6 +192,19 @@ struct TileLoader {
     }
 };
 
+// Position of this block when each XCD takes a contiguous range of the
+// launch's (split, tile) sequence.  Blocks go round-robin over the 8 XCDs in
+// order of their linear id, so ids x, x + 8, .. of a launch share an L2: XCD
+// x gets the x-th of 8 ranges (the first total % 8 one longer).  Over a
+// split-K grid an XCD so works few splits and reads a fraction of K of both
+// operands, where one range of tiles for every split would have each XCD
+// read all of K.
+__device__ __forceinline__ int xcd_band() {
+    const int total = gridDim.x * gridDim.z, lin = blockIdx.z * gridDim.x + blockIdx.x;
+    const int q = total >> 3, r = total & 7, x = lin & 7;
+    return x * q + min(x, r) + (lin >> 3);
+}
+
 template <int BM, int BN, int WM, int WN, bool XK, bool YK, int EPI>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) {
     constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
@@ -203,12 +216,11 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) 
 
     // XCD-aware block order: hardware dispatches consecutive block ids
     // round-robin over 8 XCDs; give each XCD a contiguous band of tiles.
-    int nt = a.tiles_m * a.tiles_n;
-    int bid = blockIdx.x;
-    if ((nt & 7) == 0) bid = (bid & 7) * (nt >> 3) + (bid >> 3);
-    int tm_i = bid / a.tiles_n, tn_i = bid % a.tiles_n;
+    const int bid = xcd_band();
+    const int nt = a.tiles_m * a.tiles_n, zs = bid / nt, tile = bid - zs * nt;
+    int tm_i = tile / a.tiles_n, tn_i = tile % a.tiles_n;
     int m0 = tm_i * BM, n0 = tn_i * BN;
-    int kbeg = blockIdx.z * a.k_per_split;
+    int kbeg = zs * a.k_per_split;
     int kend = min(a.K, kbeg + a.k_per_split);
 
     int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -290,7 +302,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) 
                     if (a.beta != 0.f) o += a.beta * (*C);
                     *C = o;
                 } else {
-                    a.part[((int64_t)blockIdx.z * a.M + m) * a.N + n] = v;
+                    a.part[((int64_t)zs * a.M + m) * a.N + n] = v;
                 }
             }
         }
@@ -307,12 +319,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // tiles at once) measured 0.4% faster on the c3 step than 4 (4 x 8) and
 // 1% faster than 16.
 constexpr int TILE_GM = 8;
-__device__ __forceinline__ void big_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    int nt = tiles_m * tiles_n;
-    if ((nt & 7) == 0) bid = (bid & 7) * (nt >> 3) + (bid >> 3);
-    int gsz = TILE_GM * tiles_n;
+__device__ __forceinline__ void big_tile(const GemmArgs& a, int& tm, int& tn, int& zs) {
+    const int nt = a.tiles_m * a.tiles_n;
+    int bid = xcd_band();
+    zs = bid / nt;
+    bid -= zs * nt;
+    int gsz = TILE_GM * a.tiles_n;
     int g = bid / gsz, idx = bid % gsz;
-    int rows = min(TILE_GM, tiles_m - g * TILE_GM);
+    int rows = min(TILE_GM, a.tiles_m - g * TILE_GM);
     tm = g * TILE_GM + idx % rows;
     tn = idx / rows;
 }
@@ -334,7 +348,7 @@ __device__ __attribute__((always_inline)) inline void big_epilogue(floatx16 (&ac
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     int m = m0 + wm * WTM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (m < a.M) a.part[((int64_t)blockIdx.z * a.M + m) * a.N + n] = acc[i][j][r];
+                    if (m < a.M) a.part[(int64_t)m * a.N + n] = acc[i][j][r];
                 }
             }
     } else {
@@ -674,9 +688,11 @@ __global__ __launch_bounds__(WMW * WNW * 64) void k_gemm_dma(GemmArgs a) {
     __shared__ __attribute__((aligned(1024))) bf16 sX4[NS == 5 ? SX : 16], sY4[NS == 5 ? SY : 16];
 
     int tm_i, tn_i;
-    big_tile(blockIdx.x, a.tiles_m, a.tiles_n, tm_i, tn_i);
+    int zs;
+    big_tile(a, tm_i, tn_i, zs);
     int m0 = tm_i * BM, n0 = tn_i * BN;
-    int kbeg = blockIdx.z * a.k_per_split;
+    int kbeg = zs * a.k_per_split;
+    if constexpr (EPI == EPI_PARTIAL) a.part += (int64_t)zs * a.M * a.N;
     int kend = min(a.K, kbeg + a.k_per_split);
     int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int wm = w / WNW, wn = w % WNW;
@@ -787,6 +803,39 @@ __device__ __forceinline__ void pipe_frags(Frags<TM, TN>& f, const bf16* sX, con
         int R = wn * WTN + j * 32 + (lane & 31);
         f.b[j] = *(const bf16x8_t*)(sY + R * KD + 8 * (c ^ stage_swz<KD>(R)));
     }
+}
+
+// pipe_frags with the lane's byte offsets into a stage precomputed (they do
+// not depend on the stage): one add per fragment and step of a loop whose
+// buffer is not known at compile time.
+template <int TM, int TN>
+struct FragOffs {
+    uint32_t a[4][TM], b[4][TN];
+};
+template <int TM, int TN, int WTM, int WTN, int KD>
+__device__ __forceinline__ void frag_offsets(FragOffs<TM, TN>& o, int wm, int wn, int lane) {
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+        const int c = 2 * kk + (lane >> 5);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const int R = wm * WTM + i * 32 + (lane & 31);
+            o.a[kk][i] = 2 * (R * KD + 8 * (c ^ stage_swz<KD>(R)));
+        }
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int R = wn * WTN + j * 32 + (lane & 31);
+            o.b[kk][j] = 2 * (R * KD + 8 * (c ^ stage_swz<KD>(R)));
+        }
+    }
+}
+template <int TM, int TN>
+__device__ __forceinline__ void pipe_frags_at(Frags<TM, TN>& f, const FragOffs<TM, TN>& o,
+                                              const bf16* sX, const bf16* sY, int kk) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) f.a[i] = *(const bf16x8_t*)((const char*)sX + o.a[kk][i]);
+#pragma unroll
+    for (int j = 0; j < TN; j++) f.b[j] = *(const bf16x8_t*)((const char*)sY + o.b[kk][j]);
 }
 
 // The accumulators hold the transposed fragments (Y rows as the MFMA's A
@@ -1083,13 +1132,18 @@ __device__ __forceinline__ void ce_frags(bf16x8_t (&fa)[TM], int kt, int kk, con
 // CEX: X holds logits and the MFMAs take dlogits formed from them (ce_frags).
 // PART: split-K, split blockIdx.z over k [z k_per_split, +k_per_split): F32
 // partials of the split into part[z][M][N], no epilogue arithmetic.
+// DEEP: 128-row tiles with DEEP stages of 64 k in flight, loaded by PW waves
+// of their own (0: the two-stage loop, loaded by the computing waves); see
+// k_gemm_deep.
 template <int BN, int WMW, int WNW, bool CHAIN, bool SWIGLU = false, int KD = 32, int BM = 256,
-          bool CEX = false, bool PART = false>
+          bool CEX = false, bool PART = false, int DEEP = 0, int PW = 0>
 __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmArgs& a0) {
     static_assert(!CEX || (KD == 64 && !CHAIN && !SWIGLU), "CE operand form");
     static_assert(!PART || (KD == 64 && !CHAIN && !SWIGLU && !CEX), "split-K partials form");
     static_assert(KD == 32 || KD == 64, "stage depth");
-    constexpr int NS = KD == 32 ? 4 : 2, NW = WMW * WNW;
+    static_assert(DEEP == 0 || (KD == 64 && BM == 128 && !SWIGLU && !CEX), "deep form");
+    constexpr int NS = DEEP ? DEEP : KD == 32 ? 4 : 2, NW = WMW * WNW;
+    constexpr int LW = DEEP ? PW : NW;  // waves that load the stages
     constexpr int WTM = BM / WMW, WTN = BN / WNW;
     constexpr int TM = WTM / 32, TN = WTN / 32;
     static_assert(TM * 32 == WTM && TN * 32 == WTN && TM % 2 == 0, "wave tile");
@@ -1098,7 +1152,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
     static_assert(KD == 32 || NW == 8 || BM == 128, "64-k stages: 8-wave layouts");
     // DMA instructions per stage per wave
     constexpr int RPI = 64 / (KD / 8);  // stage rows per DMA instruction
-    constexpr int LPS = (BM / RPI + NW - 1) / NW + (BN / RPI + NW - 1) / NW;
+    constexpr int LPS = (BM / RPI + LW - 1) / LW + (BN / RPI + LW - 1) / LW;
     constexpr int SX = BM * KD, SY = BN * KD;
     static_assert(BN == 192 || BN == 256 || (BM == 128 && (BN == 64 || BN == 128)),
                   "tile width");
@@ -1110,14 +1164,16 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
     bf16* const sY1 = sYs[1];
     // epilogue operands staged at the start: rank-16 LoRA U/V rows of the
     // first LP pairs and 512 bias entries (one DMA instruction)
-    // (128 x 128 tiles stage one pair, so two blocks fit a CU's LDS)
-    constexpr int LP = (BN == 256 || (BM == 128 && BN == 128)) ? 1 : 3;
+    // (128 x 128 tiles stage one pair, so two blocks fit a CU's LDS; the deep
+    // form runs one block per CU)
+    constexpr int LP = (BN == 256 || (BM == 128 && BN == 128 && DEEP == 0)) ? 1 : 3;
     constexpr int LPU = SWIGLU ? 2 : LP;  // U rows: both pairs' h in the SwiGLU form
     static_assert(!SWIGLU || (BN == 256 && WNW == 4 && WMW == 2), "SwiGLU tile layout");
     __shared__ __attribute__((aligned(16))) bf16 sLU[LPU * BM * 16], sLV[LP * BN * 16], sB[512];
 
     int tm_i, tn_i;
-    big_tile(blockIdx.x, a0.tiles_m, a0.tiles_n, tm_i, tn_i);
+    int zs;  // split (PART)
+    big_tile(a0, tm_i, tn_i, zs);
     // N-concatenated groups: this tile's group supplies Y, C, N, bias, LoRA
     GemmArgs a = a0;
     if (a0.ngroups > 1) {
@@ -1136,7 +1192,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
     if constexpr (PART) {
         // the split's K range is the whole K of operands that start at its
         // first k (both are K-contiguous, k_per_split a multiple of 64)
-        const int k0 = blockIdx.z * a0.k_per_split;
+        const int k0 = zs * a0.k_per_split;
         a.X += k0;
         a.Y += k0;
         a.K = min(a0.K - k0, a0.k_per_split);
@@ -1187,7 +1243,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
             }
             __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)dst, 16, 0, 0);
         }
-    } else if (lds_lora) {
+    } else if (lds_lora && w < NW) {
         // instruction q moves 32 rows x 32 bytes: lane l -> row l/2, half l%2
         constexpr int UI = BM / 32, VI = BN / 32;
         for (int q = w; q < LP * (UI + VI); q += NW) {
@@ -1231,15 +1287,16 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
     // K segments: stage kt (global k) belongs to segment s; the accumulators
     // are rounded after the last stage of every segment but the last
     const int kb1 = CHAIN ? a.kseg[1] / KD : -99, kb2 = CHAIN && a.nseg > 2 ? a.kseg[2] / KD : -99;
-    DmaOffs<BM, NW, KD> ox0, ox1, ox2;
-    DmaOffs<BN, NW, KD> oy0, oy1, oy2;
+    const int lw = DEEP ? w - NW : w;  // loading wave
+    DmaOffs<BM, LW, KD> ox0, ox1, ox2;
+    DmaOffs<BN, LW, KD> oy0, oy1, oy2;
     if constexpr (CHAIN) {
-        dma_offsets<BM, NW>(ox0, a.sldx[0], m0, a.M, w, lane);
-        dma_offsets<BN, NW>(oy0, a.sldy[0], n0, a.N, w, lane);
-        dma_offsets<BM, NW>(ox1, a.sldx[1], m0, a.M, w, lane);
-        dma_offsets<BN, NW>(oy1, a.sldy[1], n0, a.N, w, lane);
-        dma_offsets<BM, NW>(ox2, a.nseg > 2 ? a.sldx[2] : 0, m0, a.M, w, lane);
-        dma_offsets<BN, NW>(oy2, a.nseg > 2 ? a.sldy[2] : 0, n0, a.N, w, lane);
+        dma_offsets<BM, LW>(ox0, a.sldx[0], m0, a.M, lw, lane);
+        dma_offsets<BN, LW>(oy0, a.sldy[0], n0, a.N, lw, lane);
+        dma_offsets<BM, LW>(ox1, a.sldx[1], m0, a.M, lw, lane);
+        dma_offsets<BN, LW>(oy1, a.sldy[1], n0, a.N, lw, lane);
+        dma_offsets<BM, LW>(ox2, a.nseg > 2 ? a.sldx[2] : 0, m0, a.M, lw, lane);
+        dma_offsets<BN, LW>(oy2, a.nseg > 2 ? a.sldy[2] : 0, n0, a.N, lw, lane);
     }
     // each segment's operands at the tile's first row (wave-uniform)
     const bf16* xt0 = CHAIN ? a.sX[0] + (int64_t)m0 * a.sldx[0] : nullptr;
@@ -1263,18 +1320,18 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
             y_ = s_ == 2 ? yt2 : s_ == 1 ? yt1 : yt0;                                      \
             k_ -= s_ == 2 ? a.kseg[2] : s_ == 1 ? a.kseg[1] : 0;                           \
             if (z_) {                                                                      \
-                if (DOX) dma_stage<BM, NW, KD>(g_dma_zero, 0, m0, a.M, 0, SXB, w, lane);            \
-                if (DOY) dma_stage<BN, NW, KD>(g_dma_zero, 0, n0, a.N, 0, SYB, w, lane);            \
+                if (DOX) dma_stage<BM, LW, KD>(g_dma_zero, 0, m0, a.M, 0, SXB, lw, lane);            \
+                if (DOY) dma_stage<BN, LW, KD>(g_dma_zero, 0, n0, a.N, 0, SYB, lw, lane);            \
             } else {                                                                       \
-                if (DOX) dma_stage_at<BM, NW, KD>(x_ + k_, s_ == 2 ? ox2 : s_ == 1 ? ox1 : ox0, SXB, \
-                                         w);                                               \
-                if (DOY) dma_stage_at<BN, NW, KD>(y_ + k_, s_ == 2 ? oy2 : s_ == 1 ? oy1 : oy0, SYB, \
-                                         w);                                               \
+                if (DOX) dma_stage_at<BM, LW, KD>(x_ + k_, s_ == 2 ? ox2 : s_ == 1 ? ox1 : ox0, SXB, \
+                                         lw);                                               \
+                if (DOY) dma_stage_at<BN, LW, KD>(y_ + k_, s_ == 2 ? oy2 : s_ == 1 ? oy1 : oy0, SYB, \
+                                         lw);                                               \
             }                                                                              \
         } else {                                                                           \
-            if (DOX) dma_stage<BM, NW, KD>(z_ ? g_dma_zero : x_, z_ ? 0 : lx_, m0, a.M, k_, SXB, w, \
+            if (DOX) dma_stage<BM, LW, KD>(z_ ? g_dma_zero : x_, z_ ? 0 : lx_, m0, a.M, k_, SXB, lw, \
                                   lane);                                                   \
-            if (DOY) dma_stage<BN, NW, KD>(z_ ? g_dma_zero : y_, z_ ? 0 : ly_, n0, a.N, k_, SYB, w, \
+            if (DOY) dma_stage<BN, LW, KD>(z_ ? g_dma_zero : y_, z_ ? 0 : ly_, n0, a.N, k_, SYB, lw, \
                                   lane);                                                   \
         }                                                                                  \
     } while (0)
@@ -1287,8 +1344,64 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         if constexpr (CHAIN)                                                               \
             if ((KT) + 1 == kb1 || (KT) + 1 == kb2) round_acc<TM, TN>(acc);                \
     } while (0)
-    Frags<TM, TN> f0, f1;
-    if constexpr (KD == 32) {
+    [[maybe_unused]] Frags<TM, TN> f0, f1;
+    if constexpr (DEEP > 0) {
+    if (w >= NW) {
+        // loading waves: stages 0 .. NS - 1, then stage kt + NS into the
+        // buffer of stage kt at the barrier after which every wave has read
+        // it.  Each step's barrier also says that stage kt + 1 has landed:
+        // while stages remain to be issued the NS - 2 after it may stay in
+        // flight.
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+            if (q < nk) PIPE_ISSUE(sXs[q], sYs[q], q);
+        if (nk >= NS)
+            TA_WAIT_VMCNT(LPS * (NS - 1));
+        else
+            TA_WAIT_VMCNT(0);
+        __builtin_amdgcn_s_barrier();
+        for (int kt = 0, b = 0; kt < nk; kt++, b = b + 1 == NS ? 0 : b + 1) {
+            if (kt + NS - 1 < nk)
+                TA_WAIT_VMCNT(LPS * (NS - 2));
+            else
+                TA_WAIT_VMCNT(0);
+            __builtin_amdgcn_s_barrier();
+            if (kt + NS < nk) PIPE_ISSUE(&sXs[0][0] + b * SX, &sYs[0][0] + b * SY, kt + NS);
+        }
+        TA_WAIT_VMCNT(0);
+        __syncthreads();  // the one before the epilogue
+        return;
+    }
+    __builtin_amdgcn_s_barrier();
+    FragOffs<TM, TN> fo;
+    frag_offsets<TM, TN, WTM, WTN, KD>(fo, wm, wn, lane);
+    Frags<TM, TN> fa[4], fb[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) pipe_frags_at<TM, TN>(fa[kk], fo, sX0, sY0, kk);
+    // step kt, its fragments in FC: wait until this wave's LDS reads (stage
+    // kt's) are done, barrier, then read stage kt + 1's fragments (buffer nb)
+    // into FN under the MFMAs
+#define DEEP_STEP(KT, FC, FN)                                                              \
+    {                                                                                      \
+        nb = nb + 1 == NS ? 0 : nb + 1;                                                    \
+        const bf16 *const SXN = &sXs[0][0] + nb * SX, *const SYN = &sYs[0][0] + nb * SY;   \
+        __builtin_amdgcn_s_waitcnt(0xc07f); /* lgkmcnt(0) */                               \
+        __builtin_amdgcn_s_barrier();                                                      \
+        _Pragma("unroll") for (int kk = 0; kk < 4; kk++) {                                 \
+            pipe_frags_at<TM, TN>(FN[kk], fo, SXN, SYN, kk);                               \
+            pipe_mma<TM, TN>(acc, FC[kk]);                                                 \
+            pipe_interleave<TM * TN, TM + TN>();                                           \
+        }                                                                                  \
+        PIPE_ROUND(KT);                                                                    \
+        if ((KT) + 1 >= nk) break;                                                         \
+    }
+    int nb = 0;
+    for (int kt = 0; kt < nk; kt += 2) {
+        DEEP_STEP(kt, fa, fb)
+        DEEP_STEP(kt + 1, fb, fa)
+    }
+#undef DEEP_STEP
+    } else if constexpr (KD == 32) {
     bf16* const sX2 = sXs[2];
     bf16* const sX3 = sXs[3];
     bf16* const sY2 = sYs[2];
@@ -1389,7 +1502,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         __syncthreads();  // every wave is done with the stage buffers
         float* const st = (float*)(w < NXR ? (char*)&sXs[0][0] + w * RB
                                            : (char*)&sYs[0][0] + (w - NXR) * RB);
-        float* const P = a0.part + (int64_t)blockIdx.z * a0.M * a0.N;
+        float* const P = a0.part + (int64_t)zs * a0.M * a0.N;
         const bool v4 = (a0.N & 3) == 0;
 #pragma unroll
         for (int i = 0; i < TM; i++) {
@@ -1551,6 +1664,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     gemm_pipe_body<BN, 2, 2, true, false, 64, 128>(a);
 }
 
+// k_gemm_deep: outputs of at most one 128 x BN tile per CU (BN = 64 or 128).
+// With a single block on a CU and 0.2-0.4 us of MFMAs per 64-k stage, what
+// bounds the two-stage kernel is the latency of a stage's load (about 0.8 us
+// from HBM), not its bandwidth.  Four stages stay in flight (96 or 128 KB of
+// LDS), four loading waves issue them so that no MFMA waits behind the
+// address unit's queue, and the four computing waves read a whole stage's
+// fragments while the previous stage computes.  Measured (operands from HBM,
+// us): 2048 x 896 x 896 11.5 -> 8.4, 2048 x 1536 x 1536 17.8 -> 14.7,
+// 2048 x 896 x 4864 42 (256-row split-K) -> 35, 64 x 896 x 896 25 -> 7.1.
+// Six stages of 128 x 64 measured the same; two loading waves 1-3% slower.
+constexpr int DEEP_NS = 4, DEEP_LW = 4, DEEP_THREADS = 256 + 64 * DEEP_LW;
+template <int BN>
+__global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep(
+    GemmArgs a) {
+    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, false, DEEP_NS, DEEP_LW>(a);
+}
+template <int BN>
+__global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep_chain(
+    GemmArgs a) {
+    gemm_pipe_body<BN, 2, 2, true, false, 64, 128, false, false, DEEP_NS, DEEP_LW>(a);
+}
+// split-K F32 partials (grid z = splits), reduced by splitk_reduce
+template <int BN>
+__global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep_part(
+    GemmArgs a) {
+    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, true, DEEP_NS, DEEP_LW>(a);
+}
+
 // Kernel variants of the large GEMMs (ta_gemm_rm_variant): 0 picks k_gemm_pipe
 // with 8 waves and 64-k stages (256 x 192 tiles in a 4 x 2 wave layout up
 // to N = 3072, 256 x 256 in a 2 x 4 layout above; N = 1536 then gives one
@@ -1629,6 +1770,101 @@ __global__ void k_splitk_reduce(const float* __restrict__ part, int splits, int 
     }
 }
 
+// k_splitk_reduce with four consecutive outputs of a row per thread: the
+// partials as 16-byte loads, eight splits in flight.  N and ldc multiples
+// of 4, C 8-byte (BF16) or 16-byte (F32) aligned.  Same sums in the same
+// order as the one-output form.
+template <bool OUT_BF16>
+__global__ __launch_bounds__(256) void k_splitk_reduce4(const float* __restrict__ part, int splits,
+                                                        int M, int N, void* __restrict__ Cv,
+                                                        int64_t ldc, float alpha, float beta,
+                                                        const bf16* __restrict__ bias) {
+    const int64_t idx = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
+    const int64_t MN = (int64_t)M * N;
+    if (idx >= MN) return;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    int z = 0;
+    for (; z + 8 <= splits; z += 8) {
+        float4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = *(const float4*)(part + (int64_t)(z + i) * MN + idx);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            s[0] += v[i].x;
+            s[1] += v[i].y;
+            s[2] += v[i].z;
+            s[3] += v[i].w;
+        }
+    }
+    if (z < splits) {
+        float4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (z + i < splits) v[i] = *(const float4*)(part + (int64_t)(z + i) * MN + idx);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (z + i < splits) {
+                s[0] += v[i].x;
+                s[1] += v[i].y;
+                s[2] += v[i].z;
+                s[3] += v[i].w;
+            }
+    }
+    const int m = (int)(idx / N), n = (int)(idx % N);
+    if (OUT_BF16) {
+        bf16* C = (bf16*)Cv + (int64_t)m * ldc + n;
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = alpha * s[e];
+        if (beta != 0.f) {
+            const uint2 c = *(const uint2*)C;
+            o[0] += beta * lo2f(c.x);
+            o[1] += beta * hi2f(c.x);
+            o[2] += beta * lo2f(c.y);
+            o[3] += beta * hi2f(c.y);
+        }
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = bf2f(f2bf(o[e])) + bf2f(bias[n + e]);
+        }
+        uint2 w;
+        w.x = pack2(o[0], o[1]);
+        w.y = pack2(o[2], o[3]);
+        *(uint2*)C = w;
+    } else {
+        float4* C = (float4*)((float*)Cv + (int64_t)m * ldc + n);
+        float4 o = make_float4(alpha * s[0], alpha * s[1], alpha * s[2], alpha * s[3]);
+        if (beta != 0.f) {
+            const float4 c = *C;
+            o.x += beta * c.x;
+            o.y += beta * c.y;
+            o.z += beta * c.z;
+            o.w += beta * c.w;
+        }
+        *C = o;
+    }
+}
+
+// Add the splits' partials in order into C.
+static void splitk_reduce(const float* part, int splits, int M, int N, void* C, int64_t ldc,
+                          float alpha, float beta, const bf16* bias, bool out_f32, hipStream_t s) {
+    const int64_t MN = (int64_t)M * N;
+    const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & (out_f32 ? 15u : 7u)) == 0;
+    const dim3 grid((unsigned)((MN + (v4 ? 1023 : 255)) / (v4 ? 1024 : 256)));
+    if (v4 && out_f32)
+        tlaunch(k_splitk_reduce4<false>, grid, dim3(256), s, part, splits, M, N, C, ldc, alpha, beta,
+                bias);
+    else if (v4)
+        tlaunch(k_splitk_reduce4<true>, grid, dim3(256), s, part, splits, M, N, C, ldc, alpha, beta,
+                bias);
+    else if (out_f32)
+        tlaunch(k_splitk_reduce<false>, grid, dim3(256), s, part, splits, M, N, C, ldc, alpha, beta,
+                bias);
+    else
+        tlaunch(k_splitk_reduce<true>, grid, dim3(256), s, part, splits, M, N, C, ldc, alpha, beta,
+                bias);
+}
+
 template <int BM, int BN, int WM, int WN, int EPI>
 static void launch_cfg(bool xk, bool yk, const GemmArgs& a, int splits, bool vx, bool vy,
                        hipStream_t s) {
@@ -1649,6 +1885,8 @@ static inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 constexpr int64_t kMaxStageLd = int64_t(1) << 23;
 
 // Tile width of k_gemm_mid for an M x N output (0: the 256-row kernels).
+// Asked after deep_plan, which takes the grids of at most one block per CU:
+// what is left for k_gemm_mid are 257 or more 128-row tiles.
 // The 256-row tiles stay while they fill most of the chip (big_ok: that
 // kernel can take the shape), and for long K (32 or more 64-k stages),
 // where they run split-K: 128-row tiles reread each operand band twice as
@@ -1670,12 +1908,94 @@ static int mid_bn(int M, int N, int BNb, int ksteps, bool big_ok, int n_mult) {
     if (big_ok) return 0;
     return n_mult % 128 == 0 ? 128 : n_mult % 64 == 0 ? 64 : 0;
 }
+static const char* deep_name(int bn, bool chain) {
+    if (chain)
+        return bn == 128 ? "void ta::k_gemm_deep_chain<128>(ta::GemmArgs)"
+                         : "void ta::k_gemm_deep_chain<64>(ta::GemmArgs)";
+    return bn == 128 ? "void ta::k_gemm_deep<128>(ta::GemmArgs)"
+                     : "void ta::k_gemm_deep<64>(ta::GemmArgs)";
+}
 static const char* mid_name(int bn, bool chain) {
     if (chain)
         return bn == 128 ? "void ta::k_gemm_mid_chain<128>(ta::GemmArgs)"
                          : "void ta::k_gemm_mid_chain<64>(ta::GemmArgs)";
     return bn == 128 ? "void ta::k_gemm_mid<128>(ta::GemmArgs)"
                      : "void ta::k_gemm_mid<64>(ta::GemmArgs)";
+}
+
+// whether s records into a graph (also when that cannot be told)
+static bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// F32 partials of an M x N output written and read back over `splits`: the
+// reduce's launch and the traffic at the rate it measured (GB/s).
+static double split_us(int M, int N, int splits, double gbs) {
+    return splits > 1 ? 2.0 + (double)splits * M * N * 8.0 / (gbs * 1e3) : 0.0;
+}
+
+// Tile width and K splits of k_gemm_deep for an M x N x K product (bn 0: not
+// this kernel), with the time it is expected to take.  The kernel runs one
+// block per CU, so only grids of at most 256 blocks qualify.  The model,
+// fitted to 290 measured (shape, width, splits) times (geometric mean of the
+// choice within 1.5% of the best measured one): a fixed 4.3 us (64-wide) or
+// 5 us (128-wide), and per 64-k stage 0.27 or 0.36 us on an empty chip, 45%
+// more with all 256 CUs loading; 2 us and 4 TB/s for the partials of a
+// split.  So K = 896 .. 1536 runs unsplit, and a long K over few tiles
+// splits until the partials cost what the stages gain (128 x 896 x 4864:
+// 23.2 us unsplit, 16.1, 11.9, 10.6 and 12.2 us in 2, 4, 8 and 16 splits).
+struct DeepPlan {
+    int bn = 0, splits = 1;
+    double us = 1e30;
+};
+static DeepPlan deep_plan(int M, int N, int ksteps, bool can_split, int n_mult) {
+    DeepPlan best;
+    if (N < 64) return best;
+    for (int bn = 64; bn <= 128; bn *= 2) {
+        if (n_mult % bn != 0) continue;
+        const int64_t t = (int64_t)ceil_div(M, 128) * ceil_div(N, bn);
+        if (t > 256) continue;
+        const int most = can_split ? std::max(1, std::min((int)(256 / t), ksteps / 6)) : 1;
+        // powers of two, and the count that fills the chip
+        for (int q = 1;; q = std::min(2 * q, most)) {
+            const int per = ceil_div(ksteps, q), sp = ceil_div(ksteps, per);
+            const double load = 1.0 + 0.45 * (double)t * sp / 256.0;
+            const double us = (bn == 64 ? 4.3 + 0.27 * load * per : 5.0 + 0.36 * load * per) +
+                              split_us(M, N, sp, 4000.0);
+            if (us < best.us) {
+                best.bn = bn;
+                best.splits = sp;
+                best.us = us;
+            }
+            if (q >= most) break;
+        }
+    }
+    return best;
+}
+// Expected time of the 256-row kernels on a long-K product (ksteps >= 32) of
+// `tiles` tiles in `splits` splits: 7 us and 1.35 us per 64-k stage for each
+// wave of 256 blocks, and the partials at 5.5 TB/s (measured the same way).
+// LoRA terms run as a pass of their own after a split.
+static double split256_us(int M, int N, int ksteps, int tiles, int splits, bool lora) {
+    const int per = ceil_div(ksteps, splits), sp = ceil_div(ksteps, per);
+    return (double)ceil_div(tiles * sp, 256) * (7.0 + 1.35 * per) + split_us(M, N, sp, 5500.0) +
+           (sp > 1 && lora ? 3.0 + (double)M * N * 4.0 / 2.5e6 : 0.0);
+}
+
+// Expected time of one K-contiguous GEMM of a chain or a group run as a
+// launch of its own (the faster of the two forms above).
+static double segment_us(int M, int N, int ksteps, bool lora) {
+    const DeepPlan dp = deep_plan(M, N, ksteps, true, 128);
+    const double deep = dp.us + (dp.splits > 1 && lora ? 3.0 + (double)M * N * 4.0 / 2.5e6 : 0.0);
+    const int t = ceil_div(M, 256) * ceil_div(N, 256);
+    const int sp = ksteps >= 32 ? std::max(1, std::min(256 / std::min(t, 256), ksteps / 8)) : 1;
+    return std::min(deep, split256_us(M, N, ksteps, t, sp, lora));
 }
 
 // Shape-driven dispatch.  out_f32: C is F32 (gemm_f32 semantics).  lora
@@ -1722,31 +2042,93 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     bool vx = al16(X) && (ldx % 8) == 0;
     bool vy = al16(Y) && (ldy % 8) == 0;
 
-    // K-contiguous BF16 GEMMs too small to fill the chip with 256-row tiles:
-    // k_gemm_mid (128-row tiles, LoRA terms in the epilogue)
     const bool pipe_ok = xk && yk && !out_f32 && (K % BK) == 0 && vx && vy &&
                          ldx < kMaxStageLd && ldy < kMaxStageLd;
-    if (pipe_ok && ((g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0) ||
-                    g_big_variant == 19 || g_big_variant == 20)) {
-        const bool big_ok = M >= 1024 && N >= 1024;
+    const bool lora_on = lora && lora->n > 0;
+    auto set_lora = [&]() {
+        if (!lora_on) return;
+        a.lora_n = lora->n;
+        a.lora_r = lora->r;
+        a.lora_delta = lora->delta ? 1 : 0;
+        a.lora_s = lora->s;
+        for (int p = 0; p < lora->n; p++) {
+            a.lora_u[p] = lora->u[p];
+            a.lora_ldu[p] = lora->ldu[p];
+            a.lora_v[p] = lora->v_nk[p];
+        }
+    };
+    const int ksteps = (K + BK - 1) / BK;
+    const int t192 = ((M + 255) / 256) * ((N + 191) / 192);
+    const int t256 = ((M + 255) / 256) * ((N + 255) / 256);
+    // split-K over few 256-row tiles: as many splits as keep the blocks within
+    // one per CU (at least 8 stages each), with the tile width that gives the
+    // most blocks (256-wide on a tie)
+    auto split_for = [&](int tiles) { return std::max(1, std::min(256 / tiles, ksteps / 8)); };
+    const int split_variant = t192 * split_for(t192) > t256 * split_for(t256) ? 17 : 18;
+    const bool auto_form = g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0;
+    const bool big_shape =
+        (M >= 1024 && N >= 1024) || (M >= 256 && N >= 128 && ksteps >= 32);
+    // K-contiguous BF16 GEMMs too small to fill the chip with 256-row tiles:
+    // k_gemm_deep when one 128-row tile per CU covers the output (and a long K
+    // does not run faster in the 256-row kernels' splits), else k_gemm_mid
+    // (LoRA terms in the epilogue of both)
+    if (pipe_ok && (auto_form || g_big_variant == 19 || g_big_variant == 20)) {
         const int bn = g_big_variant == 19   ? 128
                        : g_big_variant == 20 ? 64
-                                             : mid_bn(M, N, N > 3072 ? 256 : 192, K / BK, big_ok, 128);
+                                             : mid_bn(M, N, N > 3072 ? 256 : 192, ksteps,
+                                                      M >= 1024 && N >= 1024, 128);
+        DeepPlan dp;
+        if (auto_form) {
+            // (a capture of a shape that no other form splits takes no pointer
+            // into the scratch pool, which may move before a replay)
+            const bool fresh_split = M >= 128 && !(bn == 0 && big_shape);
+            dp = deep_plan(M, N, ksteps, true, 128);
+            if (dp.bn && dp.splits > 1 && fresh_split && is_capturing(s))
+                dp = deep_plan(M, N, ksteps, false, 128);
+            if (dp.bn && bn == 0 && big_shape) {
+                const int t = split_variant == 17 ? t192 : t256;
+                if (dp.us > 0.97 * split256_us(M, N, ksteps, t, split_for(t), lora_on)) dp.bn = 0;
+            }
+        }
+        if (dp.bn) {
+            a.tiles_m = (M + 127) / 128;
+            a.tiles_n = (N + dp.bn - 1) / dp.bn;
+            const int per = ceil_div(ksteps, dp.splits);
+            a.k_per_split = per * BK;
+            const dim3 grid(a.tiles_m * a.tiles_n, 1, dp.splits);
+            if (dp.splits > 1) {
+                const size_t bytes = (size_t)dp.splits * M * N * sizeof(float);
+                a.part = (float*)scratch_get(bytes, s);
+                if (!a.part)
+                    return set_error(-2, "gemm: scratch allocation of %zu bytes failed", bytes);
+                if (dp.bn == 128)
+                    tlaunch(k_gemm_deep_part<128>, grid, dim3(DEEP_THREADS), s, a);
+                else
+                    tlaunch(k_gemm_deep_part<64>, grid, dim3(DEEP_THREADS), s, a);
+                splitk_reduce(a.part, dp.splits, M, N, C, ldc, alpha, beta, bias, false, s);
+                int rc = check_launch("gemm");
+                return rc ? rc : lora_after();
+            }
+            set_lora();
+            const bool timed = kprof_begin(KP_GEMM_BIG, s);
+            if (dp.bn == 128)
+                tlaunch(k_gemm_deep<128>, grid, dim3(DEEP_THREADS), s, a);
+            else
+                tlaunch(k_gemm_deep<64>, grid, dim3(DEEP_THREADS), s, a);
+            if (timed) {
+                double mn = (double)M * N;
+                double fl = 2.0 * mn * K + 2.0 * mn * a.lora_r * a.lora_n;
+                double by = 2.0 * ((double)M * K + (double)N * K + mn * (beta != 0.f ? 2 : 1)) +
+                            2.0 * a.lora_n * (double)(M + N) * a.lora_r;
+                kprof_end(KP_GEMM_BIG, s, fl, by, deep_name(dp.bn, false));
+            }
+            return check_launch("gemm");
+        }
         if (bn) {
             a.tiles_m = (M + 127) / 128;
             a.tiles_n = (N + bn - 1) / bn;
             a.k_per_split = K;
-            if (lora && lora->n > 0) {
-                a.lora_n = lora->n;
-                a.lora_r = lora->r;
-                a.lora_delta = lora->delta ? 1 : 0;
-                a.lora_s = lora->s;
-                for (int p = 0; p < lora->n; p++) {
-                    a.lora_u[p] = lora->u[p];
-                    a.lora_ldu[p] = lora->ldu[p];
-                    a.lora_v[p] = lora->v_nk[p];
-                }
-            }
+            set_lora();
             const bool timed = kprof_begin(KP_GEMM_BIG, s);
             dim3 grid(a.tiles_m * a.tiles_n);
             if (bn == 128)
@@ -1767,9 +2149,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     // (the stage loads address 256 operand rows with 32-bit byte offsets)
     // (smaller outputs take the 256-row tiles when a variant is forced, and
     // split-K when K is long: 32 or more 64-k stages)
-    const int ksteps = (K + BK - 1) / BK;
-    if (pipe_ok && ((M >= 1024 && N >= 1024) || (M >= 256 && N >= 128 && ksteps >= 32) ||
-                    (g_big_variant != 0 && M >= 256 && N >= 128))) {
+    if (pipe_ok && (big_shape || (g_big_variant != 0 && M >= 256 && N >= 128))) {
         int variant = g_big_variant;
         if (variant == 0) variant = N > 3072 ? 18 : 17;
         // up to N = 3072 the 256-wide tiles when they need fewer waves of 256
@@ -1781,17 +2161,9 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
             const int64_t w256 = (tm * ((N + 255) / 256) + 255) / 256;
             if (w256 * 256 < w192 * 192) variant = 18;
         }
-        // split-K over few tiles: as many splits as keep the blocks within one
-        // per CU (at least 8 stages each), with the tile width that gives the
-        // most blocks (256-wide on a tie)
-        auto split_for = [&](int tiles) {
-            return std::max(1, std::min(256 / tiles, ksteps / 8));
-        };
-        const int t192 = ((M + 255) / 256) * ((N + 191) / 192);
-        const int t256 = ((M + 255) / 256) * ((N + 255) / 256);
         const bool auto_split = force_splits <= 0 && g_force_splits == 0 && ksteps >= 32;
         if (g_big_variant == 0 && auto_split && (N > 3072 ? t256 : t192) < 192)
-            variant = t192 * split_for(t192) > t256 * split_for(t256) ? 17 : 18;
+            variant = split_variant;
         const int BNb = big_bn(variant);
         a.tiles_m = (M + 255) / 256;
         a.tiles_n = (N + BNb - 1) / BNb;
@@ -1856,9 +2228,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
             else
                 launch_big<EPI_PARTIAL>(is_pipe(variant) ? (BNb == 256 ? 8 : 7) : variant, grid,
                                         a, s);
-            int64_t MN = (int64_t)M * N;
-            tlaunch(k_splitk_reduce<true>, dim3((int)((MN + 255) / 256)), dim3(256), s, a.part, splits, M, N, C,
-                                                                          ldc, alpha, beta, bias);
+            splitk_reduce(a.part, splits, M, N, C, ldc, alpha, beta, bias, false, s);
             int rc = check_launch("gemm");
             return rc ? rc : lora_after();
         }
@@ -1867,17 +2237,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         // run after the GEMM
         const bool fuse = lora && lora->n > 0 && (lora->r & 7) == 0 &&
                           (!is_pipe(variant) || lora->r <= 64);
-        if (fuse) {
-            a.lora_n = lora->n;
-            a.lora_r = lora->r;
-            a.lora_delta = lora->delta ? 1 : 0;
-            a.lora_s = lora->s;
-            for (int p = 0; p < lora->n; p++) {
-                a.lora_u[p] = lora->u[p];
-                a.lora_ldu[p] = lora->ldu[p];
-                a.lora_v[p] = lora->v_nk[p];
-            }
-        }
+        if (fuse) set_lora();
         // measurement hook: algorithmic work of the launch (MNK product,
         // rank-r epilogue products; operands read once, C written once and
         // read once more when beta != 0)
@@ -1970,14 +2330,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         TA_LAUNCH(128, 32, 4, 1);
 #undef TA_LAUNCH
     if (splits > 1) {
-        int64_t MN = (int64_t)M * N;
-        int blocks = (int)((MN + 255) / 256);
-        if (out_f32)
-            tlaunch(k_splitk_reduce<false>, dim3(blocks), dim3(256), s, a.part, splits, M, N, C, ldc, alpha,
-                                                          beta, bias);
-        else
-            tlaunch(k_splitk_reduce<true>, dim3(blocks), dim3(256), s, a.part, splits, M, N, C, ldc, alpha,
-                                                         beta, bias);
+        splitk_reduce(a.part, splits, M, N, C, ldc, alpha, beta, bias, out_f32, s);
     }
     int rc = check_launch("gemm");
     return rc ? rc : lora_after();
@@ -2020,11 +2373,25 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
         }
     }
     ok &= !lora || lora->n == 0 || (lora->r <= 64 && (lora->r & 7) == 0);
-    // 128-row tiles (k_gemm_mid_chain: two 64-k stages per trip) when the
-    // 256-row chain cannot fill the chip
-    // (long chains run per segment instead, where each takes split-K)
-    int mid = 0;
-    if (g_big_variant == 0 && ns > 1 && M >= 128 && N >= 64 && Ktot / BK < 32) {
+    // 128-row tiles when the 256-row chain cannot fill the chip:
+    // k_gemm_deep_chain with one tile per CU, for chains of 32 or more stages
+    // only where it is expected to beat a launch per segment (each with its
+    // own split-K), else k_gemm_mid_chain (two 64-k stages per trip)
+    int mid = 0, deep = 0;
+    if (g_big_variant == 0 && ns > 1 && N >= 64 && !(ok && tiles >= 192)) {
+        bool dok = !lora || lora->n == 0 || (lora->r <= 64 && (lora->r & 7) == 0);
+        double seg_us = 0.0;
+        for (int q = 0; q < ns; q++) {
+            dok &= sg[q].K % BK == 0 && al16(sg[q].X) && al16(sg[q].Y) && sg[q].ldx % 8 == 0 &&
+                   sg[q].ldy % 8 == 0 && sg[q].ldx < kMaxStageLd && sg[q].ldy < kMaxStageLd;
+            seg_us += segment_us(M, N, sg[q].K / BK, lora && lora->n > 0 && q + 1 == ns);
+        }
+        if (dok) {
+            const DeepPlan dp = deep_plan(M, N, Ktot / BK, false, 128);
+            if (dp.bn && (Ktot / BK < 32 || dp.us < seg_us)) deep = dp.bn;
+        }
+    }
+    if (!deep && g_big_variant == 0 && ns > 1 && M >= 128 && N >= 64 && Ktot / BK < 32) {
         bool mok = !lora || lora->n == 0 || (lora->r <= 64 && (lora->r & 7) == 0);
         const int nk = Ktot / 64, pad = (2 - nk % 2) % 2;
         int kb = 0;
@@ -2036,7 +2403,7 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
         }
         if (mok) mid = mid_bn(M, N, BNb, Ktot / BK, ok, 128);
     }
-    if (!ok && !mid) {
+    if (!ok && !mid && !deep) {
         for (int q = 0; q < ns; q++) {
             int rc = gemm_dispatch(true, true, M, N, sg[q].K, 1.f, sg[q].X, sg[q].ldx, sg[q].Y,
                                    sg[q].ldy, q ? 1.f : 0.f, C, ldc, nullptr, false, s, 0,
@@ -2058,8 +2425,9 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
     a.alpha = 1.f;
     a.beta = 0.f;
     a.k_per_split = Ktot;
-    a.tiles_m = mid ? (M + 127) / 128 : (M + 255) / 256;
-    a.tiles_n = mid ? (N + mid - 1) / mid : (N + BNb - 1) / BNb;
+    const int bn = deep ? deep : mid ? mid : BNb;
+    a.tiles_m = deep || mid ? (M + 127) / 128 : (M + 255) / 256;
+    a.tiles_n = (N + bn - 1) / bn;
     a.ngroups = 1;
     a.nseg = ns;
     int k = 0;
@@ -2084,7 +2452,11 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
     }
     dim3 grid(a.tiles_m * a.tiles_n);
     const bool timed = kprof_begin(KP_GEMM_CHAIN, s);
-    if (mid == 128)
+    if (deep == 128)
+        tlaunch(k_gemm_deep_chain<128>, dim3(grid), dim3(DEEP_THREADS), s, a);
+    else if (deep == 64)
+        tlaunch(k_gemm_deep_chain<64>, dim3(grid), dim3(DEEP_THREADS), s, a);
+    else if (mid == 128)
         tlaunch(k_gemm_mid_chain<128>, dim3(grid), dim3(256), s, a);
     else if (mid == 64)
         tlaunch(k_gemm_mid_chain<64>, dim3(grid), dim3(256), s, a);
@@ -2103,7 +2475,8 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
         double by = 2.0 * ((double)M * Ktot + (double)N * Ktot + mn) +
                     2.0 * a.lora_n * (double)(M + N) * a.lora_r;
         kprof_end(KP_GEMM_CHAIN, s, fl, by,
-                  mid ? mid_name(mid, true)
+                  deep  ? deep_name(deep, true)
+                  : mid ? mid_name(mid, true)
                   : KD == 64 ? (BNb == 192 ? "void ta::k_gemm_pipe_chain<192, 4, 2, 64>(ta::GemmArgs)"
                                          : "void ta::k_gemm_pipe_chain<256, 2, 4, 64>(ta::GemmArgs)")
                            : (BNb == 192 ? "void ta::k_gemm_pipe_chain<192, 4, 2>(ta::GemmArgs)"
@@ -2173,8 +2546,19 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
                      ldx < kMaxStageLd && ldy < kMaxStageLd)
                         ? mid_bn(M, Ntot, BNb, K / BK, big, nmult)
                         : 0;
-    const int TBN = mid ? mid : BNb;
-    if (!big && !mid) {
+    // one 128-row tile per CU (k_gemm_deep); a long K only where one launch is
+    // expected to beat a launch (with its own split-K) per group
+    int deep = 0;
+    if (g_big_variant == 0 && ng > 1 && lora_ok && vx && vy && (K % BK) == 0 && ldx < kMaxStageLd &&
+        ldy < kMaxStageLd && !(big && tiles >= 192)) {
+        double sep_us = 0.0;
+        for (int g = 0; g < ng; g++)
+            sep_us += segment_us(M, gr[g].N, K / BK, gr[g].lora && gr[g].lora->n > 0);
+        const DeepPlan dp = deep_plan(M, Ntot, K / BK, false, nmult);
+        if (dp.bn && (mid || dp.us < sep_us)) deep = dp.bn;
+    }
+    const int TBN = deep ? deep : mid ? mid : BNb;
+    if (!big && !mid && !deep) {
         for (int g = 0; g < ng; g++) {
             int rc = gemm_dispatch(true, true, M, gr[g].N, K, 1.f, X, ldx, gr[g].Y, ldy, 0.f,
                                    gr[g].C, gr[g].ldc, gr[g].bias, false, s, 0, gr[g].lora);
@@ -2196,7 +2580,7 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
     a.beta = 0.f;
     a.bias = gr[0].bias;
     a.k_per_split = K;
-    a.tiles_m = mid ? (M + 127) / 128 : (M + 255) / 256;
+    a.tiles_m = deep || mid ? (M + 127) / 128 : (M + 255) / 256;
     a.tiles_n = Ntot / TBN;
     a.ngroups = ng;
     a.lora_r = l0 ? l0->r : 0;
@@ -2238,7 +2622,11 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
     const int kid = BNb == 256 ? KP_GEMM_BIG_WIDE : KP_GEMM_BIG;
     const bool timed = kprof_begin(kid, s);
     dim3 grid(a.tiles_m * a.tiles_n);
-    if (mid == 128)
+    if (deep == 128)
+        tlaunch(k_gemm_deep<128>, dim3(grid), dim3(DEEP_THREADS), s, a);
+    else if (deep == 64)
+        tlaunch(k_gemm_deep<64>, dim3(grid), dim3(DEEP_THREADS), s, a);
+    else if (mid == 128)
         tlaunch(k_gemm_mid<128>, dim3(grid), dim3(256), s, a);
     else if (mid == 64)
         tlaunch(k_gemm_mid<64>, dim3(grid), dim3(256), s, a);
@@ -2263,7 +2651,8 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
                 fl += 2.0 * M * gr[g].N * a.lora_r;
                 by += 2.0 * (double)(M + gr[g].N) * a.lora_r;
             }
-        kprof_end(kid, s, fl, by, mid ? mid_name(mid, false) : big_name(variant));
+        kprof_end(kid, s, fl, by,
+                  deep ? deep_name(deep, false) : mid ? mid_name(mid, false) : big_name(variant));
     }
     return check_launch("gemm_groups");
 }

@@ -10,6 +10,9 @@
 // s_waitcnt vmcnt(n) with the other counters left free (gfx9 encoding)
 #define TA_WAIT_VMCNT(n) \
     __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+// the same with lgkmcnt(0): also every LDS and scalar read of this wave is done
+#define TA_WAIT_VMCNT_LGKM0(n) \
+    __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
 
 namespace ta {
 
