@@ -156,8 +156,8 @@ int ta_adamw_fused(float* master, uint16_t* working, float* m, float* v, float* 
  * to BF16.  gemm_f32: F32 inputs and output with F32 accuracy (cublasSgemm
  * semantics): each operand is split into three BF16 parts carrying its 24
  * significand bits and the six part products down to 2^-24 relative are
- * accumulated in F32 on the BF16 MFMA; it stages the split operands in the
- * scratch pool (at most 256 MB per call, K taken in chunks).
+ * accumulated in F32 on the BF16 MFMA; a split over K keeps its F32 partials
+ * in the scratch pool.
  * Returns -1 for M,N,K,ld <= 0 (tensor.cu:134-142). */
 int ta_gemm_bf16(int transA, int transB, int M, int N, int K, float alpha,
                  const uint16_t* A, int lda, const uint16_t* B, int ldb, float beta,

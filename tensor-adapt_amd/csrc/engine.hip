@@ -619,7 +619,7 @@ static int ga_launch(Engine* e, const GaDeferred& d) {
 static int proj_fwd(Engine* e, const bf16* W, const bf16* x, bf16* y, int in, int out,
                     const bf16* bias, const LoraEpi* lora = nullptr) {
     TIMED(TA_CAT_GEMM_FWD, gflops(e->BT, out, in), gbytes(e->BT, out, in, 2, 2, false),
-          gemm_dispatch(true, true, e->BT, out, in, 1.f, x, in, W, in, 0.f, y, out, bias, false,
+          gemm_dispatch(true, true, e->BT, out, in, 1.f, x, in, W, in, 0.f, y, out, bias,
                         e->s, 0, lora && lora->n ? lora : nullptr));
     return 0;
 }
@@ -629,7 +629,7 @@ static int proj_bwd_x(Engine* e, const bf16* Wt, const bf16* dy, bf16* dx, int o
                       float beta, const LoraEpi* lora = nullptr) {
     TIMED(TA_CAT_GEMM_DX, gflops(e->BT, in, out), gbytes(e->BT, in, out, 2, 2, beta != 0.f),
           gemm_dispatch(true, true, e->BT, in, out, 1.f, dy, out, Wt, out, beta, dx, in, nullptr,
-                        false, e->s, 0, lora && lora->n ? lora : nullptr));
+                        e->s, 0, lora && lora->n ? lora : nullptr));
     return 0;
 }
 
@@ -743,7 +743,7 @@ static int forward(Engine* e) {
     // LM head (qwen2.cu:163-175), tied to the embedding when c.tie
     TIMED(TA_CAT_LMHEAD, gflops(BT, e->V, H), gbytes(BT, e->V, H, 2, 2, false),
           gemm_dispatch(true, true, BT, e->V, H, 1.f, e->xfn, H, e->lm, H, 0.f, e->logits, e->V,
-                        nullptr, false, s, 0, nullptr));
+                        nullptr, s, 0, nullptr));
     // loss (adapt_trainer.cu:201-205): dlogits overwrite the logits in place
     // (one read and one write of BT x V BF16); the first step also counts
     // the NaN and Inf logits (adapt_trainer.cu:196-198)
@@ -773,7 +773,7 @@ static int backward(Engine* e) {
     else
         TIMED(TA_CAT_LMHEAD_BWD, gflops(BT, H, e->V), gbytes(BT, H, e->V, 2, 2, false),
               gemm_dispatch(true, true, BT, H, e->V, 1.f, e->logits, e->V, e->lmT, e->V, 0.f,
-                            e->dres, H, nullptr, false, s, 0, nullptr));
+                            e->dres, H, nullptr, s, 0, nullptr));
     TIMED(TA_CAT_NORM, 0, nrm_b,
           ta_rms_norm_bwd(e->dres, e->x_final, e->final_norm, e->final_rms, e->g_res, nullptr, 1,
                           BT, H, c.rms_eps, s));

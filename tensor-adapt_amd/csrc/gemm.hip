@@ -22,8 +22,8 @@
 // (own L2 each) works a contiguous band of output tiles.
 //
 // Epilogues: BF16 (alpha, beta, optional bias added after the first
-// rounding and rounded again — the reference's gemm + ops::add_bias), F32
-// (gemm_f32 semantics), or F32 partials for split-K with a separate
+// rounding and rounded again — the reference's gemm + ops::add_bias) or F32
+// partials for split-K with a separate
 // fixed-order reduction (deterministic).
 #include <algorithm>
 #include <numeric>
@@ -50,7 +50,7 @@ __device__ __forceinline__ void st_out16(void* p, const bf16x8v& v) {
 constexpr int BK = 64;
 constexpr int LDS_STRIDE = BK + 8;  // bf16 elements per LDS row
 
-enum Epi { EPI_BF16 = 0, EPI_F32 = 1, EPI_PARTIAL = 2 };
+enum Epi { EPI_BF16 = 0, EPI_PARTIAL = 2 };
 
 struct GemmArgs {
     int M, N, K;
@@ -192,19 +192,6 @@ struct TileLoader {
     }
 };
 
-// Position of this block when each XCD takes a contiguous range of the
-// launch's (split, tile) sequence.  Blocks go round-robin over the 8 XCDs in
-// order of their linear id, so ids x, x + 8, .. of a launch share an L2: XCD
-// x gets the x-th of 8 ranges (the first total % 8 one longer).  Over a
-// split-K grid an XCD so works few splits and reads a fraction of K of both
-// operands, where one range of tiles for every split would have each XCD
-// read all of K.
-__device__ __forceinline__ int xcd_band() {
-    const int total = gridDim.x * gridDim.z, lin = blockIdx.z * gridDim.x + blockIdx.x;
-    const int q = total >> 3, r = total & 7, x = lin & 7;
-    return x * q + min(x, r) + (lin >> 3);
-}
-
 template <int BM, int BN, int WM, int WN, bool XK, bool YK, int EPI>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) {
     constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
@@ -296,11 +283,6 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) 
                     if (a.beta != 0.f) o += a.beta * bf2f(*C);
                     if (a.bias) o = bf2f(f2bf(o)) + bf2f(a.bias[n]);
                     *C = f2bf(o);
-                } else if (EPI == EPI_F32) {
-                    float* C = (float*)a.C + (int64_t)m * a.ldc + n;
-                    float o = a.alpha * v;
-                    if (a.beta != 0.f) o += a.beta * (*C);
-                    *C = o;
                 } else {
                     a.part[((int64_t)zs * a.M + m) * a.N + n] = v;
                 }
@@ -1846,7 +1828,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce4(const float* __restrict_
 }
 
 // Add the splits' partials in order into C.
-static void splitk_reduce(const float* part, int splits, int M, int N, void* C, int64_t ldc,
+void splitk_reduce(const float* part, int splits, int M, int N, void* C, int64_t ldc,
                           float alpha, float beta, const bf16* bias, bool out_f32, hipStream_t s) {
     const int64_t MN = (int64_t)M * N;
     const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & (out_f32 ? 15u : 7u)) == 0;
@@ -1998,13 +1980,12 @@ static double segment_us(int M, int N, int ksteps, bool lora) {
     return std::min(deep, split256_us(M, N, ksteps, t, sp, lora));
 }
 
-// Shape-driven dispatch.  out_f32: C is F32 (gemm_f32 semantics).  lora
-// (may be NULL): rank-r terms applied to C after the base epilogue, fused
+// Shape-driven dispatch.  lora (may be NULL): rank-r terms applied to C after the base epilogue, fused
 // into the large-GEMM kernel's epilogue when that kernel runs unsplit and
 // applied by k_rank_update right after the GEMM otherwise.
 int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16* X, int64_t ldx,
                   const bf16* Y, int64_t ldy, float beta, void* C, int64_t ldc, const bf16* bias,
-                  bool out_f32, hipStream_t s, int force_splits, const LoraEpi* lora) {
+                  hipStream_t s, int force_splits, const LoraEpi* lora) {
     GemmArgs a{};
     a.M = M;
     a.N = N;
@@ -2030,7 +2011,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     a.ngroups = 1;
     a.nseg = 1;
     if (lora && lora->n > 0) {
-        if (out_f32 || lora->n > 3 || (lora->r & 7) != 0)
+        if (lora->n > 3 || (lora->r & 7) != 0)
             return set_error(-1, "gemm: unsupported LoRA epilogue (n=%d r=%d)", lora->n, lora->r);
     }
     // runs the LoRA terms as a separate pass when the kernel did not fuse them
@@ -2042,7 +2023,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     bool vx = al16(X) && (ldx % 8) == 0;
     bool vy = al16(Y) && (ldy % 8) == 0;
 
-    const bool pipe_ok = xk && yk && !out_f32 && (K % BK) == 0 && vx && vy &&
+    const bool pipe_ok = xk && yk && (K % BK) == 0 && vx && vy &&
                          ldx < kMaxStageLd && ldy < kMaxStageLd;
     const bool lora_on = lora && lora->n > 0;
     auto set_lora = [&]() {
@@ -2182,7 +2163,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         // the last whole wave of 256-wide tiles go to k_gemm_mid.  Every
         // output element keeps its k order, so the result is the same.
         if (g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0 && splits == 1 &&
-            variant == 18 && !out_f32) {
+            variant == 18) {
             const int full = tiles / 256, rem = tiles % 256;
             if (full >= 1 && rem > 0 && rem <= 128 && (full * 256) % a.tiles_m == 0) {
                 const int n_main = full * 256 / a.tiles_m * 256;
@@ -2198,12 +2179,12 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
                         }
                     }
                     int rc = gemm_dispatch(xk, yk, M, n_main, K, alpha, X, ldx, Y, ldy, beta, C,
-                                           ldc, bias, false, s, 0, lora);
+                                           ldc, bias, s, 0, lora);
                     if (rc) return rc;
                     return gemm_dispatch(xk, yk, M, N - n_main, K, alpha, X, ldx,
                                          Y + (int64_t)n_main * ldy, ldy, beta,
                                          (bf16*)C + n_main, ldc, bias ? bias + n_main : nullptr,
-                                         false, s, 0, fz ? &lt : nullptr);
+                                         s, 0, fz ? &lt : nullptr);
                 }
             }
         }
@@ -2311,14 +2292,12 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         if (!a.part) return set_error(-2, "gemm: scratch allocation of %zu bytes failed", bytes);
         epi = EPI_PARTIAL;
     } else {
-        epi = out_f32 ? EPI_F32 : EPI_BF16;
+        epi = EPI_BF16;
     }
 #define TA_LAUNCH(BM_, BN_, WM_, WN_)                                                   \
     do {                                                                                \
         if (epi == EPI_BF16)                                                            \
             launch_cfg<BM_, BN_, WM_, WN_, EPI_BF16>(xk, yk, a, splits, vx, vy, s);     \
-        else if (epi == EPI_F32)                                                        \
-            launch_cfg<BM_, BN_, WM_, WN_, EPI_F32>(xk, yk, a, splits, vx, vy, s);      \
         else                                                                            \
             launch_cfg<BM_, BN_, WM_, WN_, EPI_PARTIAL>(xk, yk, a, splits, vx, vy, s);  \
     } while (0)
@@ -2330,7 +2309,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         TA_LAUNCH(128, 32, 4, 1);
 #undef TA_LAUNCH
     if (splits > 1) {
-        splitk_reduce(a.part, splits, M, N, C, ldc, alpha, beta, bias, out_f32, s);
+        splitk_reduce(a.part, splits, M, N, C, ldc, alpha, beta, bias, false, s);
     }
     int rc = check_launch("gemm");
     return rc ? rc : lora_after();
@@ -2406,7 +2385,7 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
     if (!ok && !mid && !deep) {
         for (int q = 0; q < ns; q++) {
             int rc = gemm_dispatch(true, true, M, N, sg[q].K, 1.f, sg[q].X, sg[q].ldx, sg[q].Y,
-                                   sg[q].ldy, q ? 1.f : 0.f, C, ldc, nullptr, false, s, 0,
+                                   sg[q].ldy, q ? 1.f : 0.f, C, ldc, nullptr, s, 0,
                                    q == ns - 1 ? lora : nullptr);
             if (rc) return rc;
         }
@@ -2561,7 +2540,7 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
     if (!big && !mid && !deep) {
         for (int g = 0; g < ng; g++) {
             int rc = gemm_dispatch(true, true, M, gr[g].N, K, 1.f, X, ldx, gr[g].Y, ldy, 0.f,
-                                   gr[g].C, gr[g].ldc, gr[g].bias, false, s, 0, gr[g].lora);
+                                   gr[g].C, gr[g].ldc, gr[g].bias, s, 0, gr[g].lora);
             if (rc) return rc;
         }
         return rope_after();
@@ -2737,42 +2716,6 @@ int gemm_swiglu(int M, int K, const bf16* X, int64_t ldx, const bf16* Wgu, const
     return check_launch("gemm_swiglu");
 }
 
-// Operand staging of gemm_f32.  Each F32 value is split into three BF16
-// parts, s0 = bf16(s), s1 = bf16(s - s0), s2 = bf16(s - s0 - s1), whose sum
-// carries s to about 2^-24 relative (24 bits of significand).  A product
-// a*b is formed as the six part products whose magnitude reaches 2^-24 of
-// it, a2 b0 + a1 b1 + a0 b2 + a1 b0 + a0 b1 + a0 b0 (smallest first, so the
-// F32 accumulator adds the small terms before the large ones); each part
-// product is exact in the MFMA's F32 arithmetic.  The parts are laid out
-// K-contiguous as six segments of kp columns per row (the segment q of a
-// row holds part (code >> 2q) & 3 of columns k0 .. k0 + kc, zero padded to
-// kp), so that one BF16 GEMM over K = 6 kp adds exactly those products.
-__global__ void k_split3(const float* __restrict__ S, int64_t ld, bool kcontig, int rows,
-                         int64_t k0, int kc, int kp, unsigned code, bf16* __restrict__ dst) {
-    const int64_t n = (int64_t)rows * kp;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t r, k;
-        if (kcontig) {
-            r = i / kp;
-            k = i - r * kp;
-        } else {
-            k = i / rows;
-            r = i - k * rows;
-        }
-        float v = 0.f;
-        if (k < kc) v = kcontig ? S[r * ld + k0 + k] : S[(k0 + k) * ld + r];
-        bf16 p[3];
-        p[0] = f2bf(v);
-        const float r1 = v - bf2f(p[0]);
-        p[1] = f2bf(r1);
-        p[2] = f2bf(r1 - bf2f(p[1]));
-        bf16* row = dst + r * (int64_t)(6 * kp) + k;
-#pragma unroll
-        for (int q = 0; q < 6; q++) row[(int64_t)q * kp] = p[(code >> (2 * q)) & 3u];
-    }
-}
-
 int gemm_ce_dx(int M, int N, int K, const bf16* logits, const bf16* Wt, bf16* C,
                const float* lse2, const int32_t* tgt, float inv_n, hipStream_t s) {
     TA_REQUIRE(M >= 256 && N >= 192 && K % BK == 0 && al16(logits) && al16(Wt) && al16(C) &&
@@ -2820,7 +2763,7 @@ int ta_gemm_rm(int x_kmajor, int y_kmajor, int M, int N, int K, float alpha, con
     TA_REQUIRE(M > 0 && N > 0 && K > 0 && ldx > 0 && ldy > 0 && ldc > 0,
                "gemm_rm: M/N/K and leading dims must be > 0");
     return gemm_dispatch(x_kmajor != 0, y_kmajor != 0, M, N, K, alpha, X, ldx, Y, ldy, beta, C,
-                         ldc, bias, false, (hipStream_t)stream, 0, nullptr);
+                         ldc, bias, (hipStream_t)stream, 0, nullptr);
 }
 
 int ta_gemm_rm_variant(int variant, int x_kmajor, int y_kmajor, int M, int N, int K, float alpha,
@@ -2849,43 +2792,7 @@ int ta_gemm_bf16(int transA, int transB, int M, int N, int K, float alpha, const
     TA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_bf16: M/N/K must be > 0");
     TA_REQUIRE(lda > 0 && ldb > 0 && ldc > 0, "gemm_bf16: leading dims must be > 0");
     return gemm_dispatch(!transB, transA != 0, N, M, K, alpha, B, ldb, A, lda, beta, C, ldc,
-                         nullptr, false, (hipStream_t)stream, 0, nullptr);
-}
-
-// cublasSgemm semantics (tensor.cu:168-182): F32 operands, F32 result.  The
-// operands are split into BF16 parts (k_split3) and multiplied on the BF16
-// MFMA with F32 accumulation, K in chunks whose staging stays within 256 MB;
-// each chunk after the first adds into C (beta 1), as a split-K SGEMM does.
-int ta_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const float* A, int lda,
-                const float* B, int ldb, float beta, float* C, int ldc, void* stream) {
-    TA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: M/N/K must be > 0");
-    TA_REQUIRE(lda > 0 && ldb > 0 && ldc > 0, "gemm_f32: leading dims must be > 0");
-    hipStream_t s = (hipStream_t)stream;
-    // rows of the row-major form: X = op(B) by output column j (N rows, K
-    // contiguous when !transB), Y = op(A) by output row i (M rows, K
-    // contiguous when transA); part codes pair a2 b0, a1 b1, a0 b2, a1 b0,
-    // a0 b1, a0 b0 segment by segment
-    const unsigned code_x = 0u | 1u << 2 | 2u << 4 | 0u << 6 | 1u << 8 | 0u << 10;
-    const unsigned code_y = 2u | 1u << 2 | 0u << 4 | 1u << 6 | 0u << 8 | 0u << 10;
-    const int64_t budget = (int64_t)256 << 20;
-    int64_t kc_max = budget / (12 * ((int64_t)M + N));
-    kc_max = kc_max < 32 ? 32 : (kc_max & ~(int64_t)31);
-    const int kcap = (int)std::min<int64_t>(kc_max, ((int64_t)K + 31) & ~(int64_t)31);
-    const size_t offy = ((size_t)N * 6 * kcap * 2 + 255) & ~(size_t)255;
-    bf16* x16 = (bf16*)scratch_get(offy + (size_t)M * 6 * kcap * 2, s, 1);
-    TA_REQUIRE(x16, "gemm_f32: scratch allocation failed");
-    bf16* y16 = (bf16*)((char*)x16 + offy);
-    for (int64_t k0 = 0; k0 < K; k0 += kcap) {
-        const int kc = (int)std::min<int64_t>(kcap, K - k0);
-        const int kp = (kc + 31) & ~31;
-        const int64_t nx = (int64_t)N * kp, ny = (int64_t)M * kp;
-        tlaunch(k_split3, dim3((int)std::min<int64_t>((nx + 255) / 256, 4096)), dim3(256), s, B, ldb, transB == 0, N, k0, kc, kp, code_x, x16);
-        tlaunch(k_split3, dim3((int)std::min<int64_t>((ny + 255) / 256, 4096)), dim3(256), s, A, lda, transA != 0, M, k0, kc, kp, code_y, y16);
-        const int rc = gemm_dispatch(true, true, N, M, 6 * kp, alpha, x16, 6 * kp, y16, 6 * kp,
-                                     k0 == 0 ? beta : 1.f, C, ldc, nullptr, true, s, 0, nullptr);
-        if (rc != 0) return rc;
-    }
-    return check_launch("gemm_f32");
+                         nullptr, (hipStream_t)stream, 0, nullptr);
 }
 
 }  // extern "C"

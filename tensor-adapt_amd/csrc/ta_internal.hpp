@@ -94,6 +94,19 @@ __device__ __forceinline__ float sum_splits(const float* __restrict__ part, int 
     return s;
 }
 
+// Position of this block when each XCD takes a contiguous range of the
+// launch's (split, tile) sequence.  Blocks go round-robin over the 8 XCDs in
+// order of their linear id, so ids x, x + 8, .. of a launch share an L2: XCD
+// x gets the x-th of 8 ranges (the first total % 8 one longer).  Over a
+// split-K grid an XCD so works few splits and reads a fraction of K of both
+// operands, where one range of tiles for every split would have each XCD
+// read all of K.
+__device__ __forceinline__ int xcd_band() {
+    const int total = gridDim.x * gridDim.z, lin = blockIdx.z * gridDim.x + blockIdx.x;
+    const int q = total >> 3, r = total & 7, x = lin & 7;
+    return x * q + min(x, r) + (lin >> 3);
+}
+
 // LoRA terms for gemm_dispatch.  After the base epilogue, for each pair p
 // in order, with D_p = U_p V_p^T (U_p [M x r], V_p [N x r]):
 //   delta: C = bf16(C + s * bf16(D_p))   (apply_lora_fwd's add)
@@ -112,7 +125,11 @@ struct LoraEpi {
 
 int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16* X, int64_t ldx,
                   const bf16* Y, int64_t ldy, float beta, void* C, int64_t ldc, const bf16* bias,
-                  bool out_f32, hipStream_t s, int force_splits, const LoraEpi* lora);
+                  hipStream_t s, int force_splits, const LoraEpi* lora);
+// C = alpha (ordered sum of the splits' F32 partials [splits][M][N]) + beta C
+// (+ bias), BF16 or F32
+void splitk_reduce(const float* part, int splits, int M, int N, void* C, int64_t ldc, float alpha,
+                   float beta, const bf16* bias, bool out_f32, hipStream_t s);
 // one of up to three GEMMs sharing X in gemm_groups: C = bf16(X Y^T (+ bias))
 // (+ LoRA delta), N output columns, row stride ldc
 struct GemmGroup {
