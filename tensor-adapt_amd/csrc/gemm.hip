@@ -29,12 +29,12 @@
 #include <numeric>
 #include <type_traits>
 
+#include "lds_tr.hpp"
 #include "ta_backend.h"
 #include "ta_internal.hpp"
 
 namespace ta {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -621,6 +621,32 @@ __device__ __forceinline__ void dma_stage_at(const bf16* __restrict__ base,
     }
 }
 
+// A 64-k stage of a K-strided operand (Y(k, n) at Y[k ldy + n]): COLS columns
+// from col0 of the 64 rows at P, kept as [64 k][COLS], one 1 KB instruction
+// per 8 (COLS = 64) or 4 (128) rows.  The MFMA's eight consecutive k of a
+// column come out of it through the transposing read (tr_frag32); one
+// 32-lane phase of that reads 64 bytes of each of four rows, so the 64-byte
+// units of a row are XOR-permuted by row bits that put the four in distinct
+// banks.  Columns past the last (cols a multiple of 8) repeat the last eight.
+template <int COLS>
+__device__ __forceinline__ int tswz(int k) {  // on the 16-byte chunk index
+    return COLS == 64 ? 4 * ((k >> 1) & 1) : 4 * (k & 3);
+}
+template <int COLS, int NW>
+__device__ __forceinline__ void dma_stage_t(const bf16* __restrict__ P, int64_t ld, int col0,
+                                            int cols, bf16* stage, int w, int lane) {
+    constexpr int LPR = COLS / 8, RPI = 64 / LPR, NI = 64 / RPI, PER = (NI + NW - 1) / NW;
+    static_assert(NI % NW == 0, "whole instructions per wave");
+#pragma unroll
+    for (int h = 0; h < PER; h++) {
+        const int j = w + NW * h, k = RPI * j + lane / LPR;
+        const int c = (lane % LPR) ^ tswz<COLS>(k);
+        const uint32_t off =
+            (uint32_t)((int64_t)k * ld * 2) + 2u * (uint32_t)(min(col0 + 8 * c, cols - 8));
+        dma16(P, off, stage + RPI * j * COLS);
+    }
+}
+
 // One 32-wide k slice of MFMAs for a wave from a swizzled stage.
 template <int TM, int TN, int WTM, int WTN>
 __device__ __attribute__((always_inline)) inline void dma_mma(floatx16 (&acc)[TM][TN],
@@ -790,12 +816,15 @@ __device__ __forceinline__ void pipe_frags(Frags<TM, TN>& f, const bf16* sX, con
 // pipe_frags with the lane's byte offsets into a stage precomputed (they do
 // not depend on the stage): one add per fragment and step of a loop whose
 // buffer is not known at compile time.
-template <int TM, int TN>
+// YT: Y's stage is [64 k][BN] (dma_stage_t); a lane's two transposing reads
+// of columns 32 j + 16 (g % 2) .. + 15 (g = l / 16) fetch rows 8 (g / 2) + 0 ..
+// 3 and + 4 .. 7 of the k step (b2 is the second).
+template <int TM, int TN, bool YT>
 struct FragOffs {
-    uint32_t a[4][TM], b[4][TN];
+    uint32_t a[4][TM], b[4][TN], b2[YT ? 4 : 1][TN];
 };
-template <int TM, int TN, int WTM, int WTN, int KD>
-__device__ __forceinline__ void frag_offsets(FragOffs<TM, TN>& o, int wm, int wn, int lane) {
+template <int TM, int TN, int WTM, int WTN, int KD, int BN, bool YT>
+__device__ __forceinline__ void frag_offsets(FragOffs<TM, TN, YT>& o, int wm, int wn, int lane) {
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) {
         const int c = 2 * kk + (lane >> 5);
@@ -806,18 +835,38 @@ __device__ __forceinline__ void frag_offsets(FragOffs<TM, TN>& o, int wm, int wn
         }
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            const int R = wn * WTN + j * 32 + (lane & 31);
-            o.b[kk][j] = 2 * (R * KD + 8 * (c ^ stage_swz<KD>(R)));
+            if constexpr (YT) {
+                const int g = lane >> 4, q = lane & 15;
+                const int k = 16 * kk + 8 * (g >> 1) + (q >> 2);
+                const int n = wn * WTN + 32 * j + 16 * (g & 1) + 4 * (q & 3);
+                o.b[kk][j] = 2 * (k * BN + (((n >> 3) ^ tswz<BN>(k)) << 3) + (n & 7));
+                o.b2[kk][j] = 2 * ((k + 4) * BN + (((n >> 3) ^ tswz<BN>(k + 4)) << 3) + (n & 7));
+            } else {
+                const int R = wn * WTN + j * 32 + (lane & 31);
+                o.b[kk][j] = 2 * (R * KD + 8 * (c ^ stage_swz<KD>(R)));
+            }
         }
     }
 }
-template <int TM, int TN>
-__device__ __forceinline__ void pipe_frags_at(Frags<TM, TN>& f, const FragOffs<TM, TN>& o,
+template <int TM, int TN, bool YT>
+__device__ __forceinline__ void pipe_frags_at(Frags<TM, TN>& f, const FragOffs<TM, TN, YT>& o,
                                               const bf16* sX, const bf16* sY, int kk) {
 #pragma unroll
     for (int i = 0; i < TM; i++) f.a[i] = *(const bf16x8_t*)((const char*)sX + o.a[kk][i]);
 #pragma unroll
-    for (int j = 0; j < TN; j++) f.b[j] = *(const bf16x8_t*)((const char*)sY + o.b[kk][j]);
+    for (int j = 0; j < TN; j++) {
+        const char* y = (const char*)sY;
+        if constexpr (YT) {
+            const i16x4_t lo =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(y + o.b[kk][j]));
+            const i16x4_t hi =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(y + o.b2[kk][j]));
+            f.b[j] = __builtin_bit_cast(bf16x8_t,
+                                        __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        } else {
+            f.b[j] = *(const bf16x8_t*)(y + o.b[kk][j]);
+        }
+    }
 }
 
 // The accumulators hold the transposed fragments (Y rows as the MFMA's A
@@ -1118,12 +1167,13 @@ __device__ __forceinline__ void ce_frags(bf16x8_t (&fa)[TM], int kt, int kk, con
 // of their own (0: the two-stage loop, loaded by the computing waves); see
 // k_gemm_deep.
 template <int BN, int WMW, int WNW, bool CHAIN, bool SWIGLU = false, int KD = 32, int BM = 256,
-          bool CEX = false, bool PART = false, int DEEP = 0, int PW = 0>
+          bool CEX = false, bool PART = false, int DEEP = 0, int PW = 0, bool YT = false>
 __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmArgs& a0) {
     static_assert(!CEX || (KD == 64 && !CHAIN && !SWIGLU), "CE operand form");
     static_assert(!PART || (KD == 64 && !CHAIN && !SWIGLU && !CEX), "split-K partials form");
     static_assert(KD == 32 || KD == 64, "stage depth");
     static_assert(DEEP == 0 || (KD == 64 && BM == 128 && !SWIGLU && !CEX), "deep form");
+    static_assert(!YT || (DEEP > 0 && !CHAIN), "K-strided Y: deep form only");
     constexpr int NS = DEEP ? DEEP : KD == 32 ? 4 : 2, NW = WMW * WNW;
     constexpr int LW = DEEP ? PW : NW;  // waves that load the stages
     constexpr int WTM = BM / WMW, WTN = BN / WNW;
@@ -1176,7 +1226,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         // first k (both are K-contiguous, k_per_split a multiple of 64)
         const int k0 = zs * a0.k_per_split;
         a.X += k0;
-        a.Y += k0;
+        a.Y += YT ? (int64_t)k0 * a.ldy : (int64_t)k0;
         a.K = min(a0.K - k0, a0.k_per_split);
         a.lora_n = 0;
         a.bias = nullptr;
@@ -1313,8 +1363,11 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         } else {                                                                           \
             if (DOX) dma_stage<BM, LW, KD>(z_ ? g_dma_zero : x_, z_ ? 0 : lx_, m0, a.M, k_, SXB, lw, \
                                   lane);                                                   \
-            if (DOY) dma_stage<BN, LW, KD>(z_ ? g_dma_zero : y_, z_ ? 0 : ly_, n0, a.N, k_, SYB, lw, \
-                                  lane);                                                   \
+            if constexpr (YT)                                                              \
+                dma_stage_t<BN, LW>(y_ + (int64_t)k_ * ly_, ly_, n0, a.N, SYB, lw, lane);  \
+            else if (DOY)                                                                  \
+                dma_stage<BN, LW, KD>(z_ ? g_dma_zero : y_, z_ ? 0 : ly_, n0, a.N, k_, SYB, \
+                                      lw, lane);                                           \
         }                                                                                  \
     } while (0)
 #define PIPE_ISSUE(SXB, SYB, KT) PIPE_ISSUE_P(SXB, SYB, KT, true, true)
@@ -1355,11 +1408,11 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         return;
     }
     __builtin_amdgcn_s_barrier();
-    FragOffs<TM, TN> fo;
-    frag_offsets<TM, TN, WTM, WTN, KD>(fo, wm, wn, lane);
+    FragOffs<TM, TN, YT> fo;
+    frag_offsets<TM, TN, WTM, WTN, KD, BN, YT>(fo, wm, wn, lane);
     Frags<TM, TN> fa[4], fb[4];
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) pipe_frags_at<TM, TN>(fa[kk], fo, sX0, sY0, kk);
+    for (int kk = 0; kk < 4; kk++) pipe_frags_at<TM, TN, YT>(fa[kk], fo, sX0, sY0, kk);
     // step kt, its fragments in FC: wait until this wave's LDS reads (stage
     // kt's) are done, barrier, then read stage kt + 1's fragments (buffer nb)
     // into FN under the MFMAs
@@ -1370,9 +1423,9 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
         __builtin_amdgcn_s_waitcnt(0xc07f); /* lgkmcnt(0) */                               \
         __builtin_amdgcn_s_barrier();                                                      \
         _Pragma("unroll") for (int kk = 0; kk < 4; kk++) {                                 \
-            pipe_frags_at<TM, TN>(FN[kk], fo, SXN, SYN, kk);                               \
+            pipe_frags_at<TM, TN, YT>(FN[kk], fo, SXN, SYN, kk);                           \
             pipe_mma<TM, TN>(acc, FC[kk]);                                                 \
-            pipe_interleave<TM * TN, TM + TN>();                                           \
+            pipe_interleave<TM * TN, TM + (YT ? 2 : 1) * TN>();                            \
         }                                                                                  \
         PIPE_ROUND(KT);                                                                    \
         if ((KT) + 1 >= nk) break;                                                         \
@@ -1657,10 +1710,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // 2048 x 896 x 4864 42 (256-row split-K) -> 35, 64 x 896 x 896 25 -> 7.1.
 // Six stages of 128 x 64 measured the same; two loading waves 1-3% slower.
 constexpr int DEEP_NS = 4, DEEP_LW = 4, DEEP_THREADS = 256 + 64 * DEEP_LW;
-template <int BN>
+// YT: Y(k, n) at Y[k ldy + n], staged as it lies and read transposed (the
+// input gradient dY W of a caller that holds W only as [out, in]).
+template <int BN, bool YT = false>
 __global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep(
     GemmArgs a) {
-    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, false, DEEP_NS, DEEP_LW>(a);
+    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, false, DEEP_NS, DEEP_LW, YT>(a);
 }
 template <int BN>
 __global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep_chain(
@@ -1668,10 +1723,59 @@ __global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2,
     gemm_pipe_body<BN, 2, 2, true, false, 64, 128, false, false, DEEP_NS, DEEP_LW>(a);
 }
 // split-K F32 partials (grid z = splits), reduced by splitk_reduce
-template <int BN>
+template <int BN, bool YT = false>
 __global__ __launch_bounds__(DEEP_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_deep_part(
     GemmArgs a) {
-    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, true, DEEP_NS, DEEP_LW>(a);
+    gemm_pipe_body<BN, 2, 2, false, false, 64, 128, false, true, DEEP_NS, DEEP_LW, YT>(a);
+}
+
+// k_gemm_rank: K <= 64, the products with a LoRA rank as their K (delta =
+// h B^T, dx += s dh A).  Two MFMAs per 16 of K and 32 x 32 outputs: bound by
+// writing C (and reading it when beta != 0), so there is no operand staging:
+// a wave loads its 64 rows of X and 64 columns of Y as fragments, and the
+// pipelined kernels' epilogue moves C as 16-byte row vectors.
+template <bool YK>
+__global__ __launch_bounds__(256) void k_gemm_rank(GemmArgs a, bool vecx, bool vecy) {
+    __shared__ __attribute__((aligned(16))) bf16 wb[4][64 * 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int m0 = (blockIdx.x % a.tiles_m) * 64, n0 = (blockIdx.x / a.tiles_m) * 256 + 64 * w;
+    if (n0 >= a.N) return;  // (no barrier below spans waves)
+    floatx16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    for (int k0 = 0; k0 < a.K; k0 += 16) {
+        const int k = k0 + 8 * (lane >> 5);
+        bf16x8_t fx[2], fy[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            fx[i] = __builtin_bit_cast(
+                bf16x8_t, load_k8(a.X, a.ldx, m0 + 32 * i + (lane & 31), k, a.M, a.K, vecx));
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int n = n0 + 32 * j + (lane & 31);
+            if constexpr (YK) {
+                fy[j] = __builtin_bit_cast(bf16x8_t, load_k8(a.Y, a.ldy, n, k, a.N, a.K, vecy));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const bool in = n < a.N && k + e < a.K;
+                    const bf16 y = a.Y[in ? (int64_t)(k + e) * a.ldy + n : 0];
+                    fy[j][e] = __builtin_bit_cast(__bf16, in ? y : (bf16)0);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fy[j], fx[i], acc[i][j], 0, 0, 0);
+    }
+    pipe_half_epilogue<2, 2, 64, 0, 1>(acc, a, (bf16*)a.C, m0, n0, lane, wb[w], nullptr, nullptr,
+                                       nullptr, 0, 0, 64, 64);
 }
 
 // Kernel variants of the large GEMMs (ta_gemm_rm_variant): 0 picks k_gemm_pipe
@@ -1894,8 +1998,8 @@ static const char* deep_name(int bn, bool chain) {
     if (chain)
         return bn == 128 ? "void ta::k_gemm_deep_chain<128>(ta::GemmArgs)"
                          : "void ta::k_gemm_deep_chain<64>(ta::GemmArgs)";
-    return bn == 128 ? "void ta::k_gemm_deep<128>(ta::GemmArgs)"
-                     : "void ta::k_gemm_deep<64>(ta::GemmArgs)";
+    return bn == 128 ? "void ta::k_gemm_deep<128, false>(ta::GemmArgs)"
+                     : "void ta::k_gemm_deep<64, false>(ta::GemmArgs)";
 }
 static const char* mid_name(int bn, bool chain) {
     if (chain)
@@ -2049,6 +2153,48 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     const bool auto_form = g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0;
     const bool big_shape =
         (M >= 1024 && N >= 1024) || (M >= 256 && N >= 128 && ksteps >= 32);
+    // K a LoRA rank (at most 64): k_gemm_rank.  The 128-row tiles below would
+    // stage 64 k of zeros and write C two bytes at a time (8192 x 1536 x 16:
+    // 22 us, and 48 us with beta 1 and a K-strided Y)
+    if (xk && K <= 64 && N >= 64 && auto_form && !lora_on) {
+        a.tiles_m = (M + 63) / 64;
+        a.tiles_n = (N + 255) / 256;
+        const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n));
+        if (yk)
+            tlaunch(k_gemm_rank<true>, grid, dim3(256), s, a, vx, vy);
+        else
+            tlaunch(k_gemm_rank<false>, grid, dim3(256), s, a, vx, vy);
+        return check_launch("gemm");
+    }
+    // K-strided Y: the same pipeline with Y staged as it lies, over as many
+    // waves of 128 x 128 tiles as the output takes (the register-staged tiles
+    // below transpose with 2-byte LDS writes: 8192 x 1536 x 1536 190 us)
+    if (xk && !yk && (K % BK) == 0 && vx && vy && N % 8 == 0 && N >= 64 && ldx < kMaxStageLd &&
+        ldy < kMaxStageLd && auto_form && !lora_on) {
+        // (as below: no scratch in a capture where the shape did not split)
+        const bool may_split = ksteps >= 16 || !is_capturing(s);
+        DeepPlan dp = deep_plan(M, N, ksteps, may_split, 128);
+        if (!dp.bn) dp.bn = 128;
+        a.tiles_m = (M + 127) / 128;
+        a.tiles_n = (N + dp.bn - 1) / dp.bn;
+        a.k_per_split = ceil_div(ksteps, dp.splits) * BK;
+        const dim3 grid(a.tiles_m * a.tiles_n, 1, dp.splits);
+        if (dp.splits > 1) {
+            const size_t bytes = (size_t)dp.splits * M * N * sizeof(float);
+            a.part = (float*)scratch_get(bytes, s);
+            if (!a.part) return set_error(-2, "gemm: scratch allocation of %zu bytes failed", bytes);
+            if (dp.bn == 128)
+                tlaunch(k_gemm_deep_part<128, true>, grid, dim3(DEEP_THREADS), s, a);
+            else
+                tlaunch(k_gemm_deep_part<64, true>, grid, dim3(DEEP_THREADS), s, a);
+            splitk_reduce(a.part, dp.splits, M, N, C, ldc, alpha, beta, bias, false, s);
+        } else if (dp.bn == 128) {
+            tlaunch(k_gemm_deep<128, true>, grid, dim3(DEEP_THREADS), s, a);
+        } else {
+            tlaunch(k_gemm_deep<64, true>, grid, dim3(DEEP_THREADS), s, a);
+        }
+        return check_launch("gemm");
+    }
     // K-contiguous BF16 GEMMs too small to fill the chip with 256-row tiles:
     // k_gemm_deep when one 128-row tile per CU covers the output (and a long K
     // does not run faster in the 256-row kernels' splits), else k_gemm_mid

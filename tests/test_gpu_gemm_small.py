@@ -49,6 +49,37 @@ def test_small_gemm(M, N, K, beta, bias):
     assert exact >= 0.9, exact
 
 
+@pytest.mark.parametrize("ykm", [0, 1])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("M,N,K,ldx,ldy", [
+    # K of a rank: k_gemm_rank (odd ranks and strides load element by element)
+    (1, 64, 2, 2, 0), (65, 257, 4, 4, 0), (64, 264, 16, 16, 0), (200, 896, 8, 24, 0),
+    (129, 100, 33, 33, 3), (2331, 1536, 64, 64, 0),
+    # K-strided Y: one tile, ragged tiles, more waves of tiles, K splits
+    (1, 64, 64, 64, 0), (130, 72, 128, 128, 8), (127, 200, 320, 320, 0), (64, 896, 4864, 4864, 0),
+    (300, 1536, 1536, 1536, 16), (2100, 4872, 192, 192, 0),
+])
+def test_rank_and_strided_gemm(M, N, K, ldx, ldy, beta, ykm):
+    """K of a LoRA rank, and Y(k, n) in rows of n (y_kmajor 0): the delta
+    h B^T, dx += s dh A and dy W of a caller that holds W as [out, in].
+    ldy is the padding of Y's rows here.  Same bound as above."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M * 5 + N + K)
+    x = rand(g, M, ldx)
+    y = rand(g, N, K + ldy, std=0.05) if ykm else rand(g, K, N + ldy, std=0.05)
+    c0 = rand(g, M, N)
+    c = c0.clone()
+    call("ta_gemm_rm", 1, ykm, M, N, K, 2.0, P(x), ldx, P(y), y.shape[1], beta, P(c), N, None, S())
+    xf = x[:, :K].float()
+    yf = (y[:, :K].t() if ykm else y[:, :N]).float()
+    want = 2.0 * (xf @ yf) + beta * c0.float()
+    mag = 2.0 * (xf.abs() @ yf.abs()) + beta * c0.float().abs()
+    err = (c.float() - want.bfloat16().float()).abs()
+    assert bool((err <= 2.0 ** -7 * want.abs() + 2.0 ** -20 * mag).all())
+    exact = float((c.float() == want.bfloat16().float()).float().mean())
+    assert exact >= 0.9 or M * N < 100, exact
+
+
 def test_small_gemm_in_a_graph():
     """A captured product gives the eager result on every replay."""
     g = torch.Generator(device=DEV)
