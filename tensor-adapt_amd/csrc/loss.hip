@@ -127,6 +127,11 @@ __device__ __forceinline__ float block_sum16(float v, float* red) {
     return r;
 }
 
+// One block per row and CU, so the phases of a row do not overlap and its VALU
+// work counts in full: two exponentials per logit, and nothing per logit that
+// a chunk can decide (the target is compared once per 8 logits; testing every
+// logit for it in two passes took 289 us at 2048 x 151,936 against 258 us, 4.8
+// TB/s, now: a large copy's rate).
 // COUNT: also add the row's NaN and Inf logits to *nonfinite (the
 // reference's step-0 check, adapt_trainer.cu:76-91)
 template <int CPT, bool COUNT>  // 16-byte chunks per lane: V <= 8 * 1024 * CPT, V % 8 == 0
@@ -137,10 +142,15 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
                                                             float inv_N,
                                                             int32_t* __restrict__ nonfinite,
                                                             float* __restrict__ lse2_out) {
-    __shared__ float red[16], tls;
+    __shared__ float red[16];
     const int64_t n = blockIdx.x;
     const bf16x8v* L = (const bf16x8v*)(logits + n * (int64_t)V);
     const int nv = V >> 3, tgt = targets[n];
+    // a target outside [0, V) reads nothing (the reference would read out of
+    // bounds for tgt >= V; ids come from a vocab-sized tokenizer)
+    const bool hit = tgt >= 0 && tgt < V;
+    // (read before the block's first barrier: dlogits may overwrite the row)
+    const float tl = hit ? bf2f(((const bf16*)L)[tgt]) : 0.f;
     bf16x8v r[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
@@ -155,12 +165,7 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
             float f[8];
             unpack8(r[k], f);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                m = fmaxf(m, f[e]);
-                // the target's logit, from the lane that holds it (dlogits may
-                // overwrite the row in place once the sums are known)
-                if (c * 8 + e == tgt) tls = f[e];
-            }
+            for (int e = 0; e < 8; e += 2) m = fmaxf(fmaxf(m, f[e]), f[e + 1]);
         }
     }
     if (COUNT) {
@@ -196,9 +201,6 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
     const float log_sum = logf(S) + M;
     const float ls2 = log_sum * kLog2e;
     if (threadIdx.x == 0) {
-        // a target outside [0, V) reads nothing (the reference would read out
-        // of bounds for tgt >= V; ids come from a vocab-sized tokenizer)
-        const float tl = (tgt >= 0 && tgt < V) ? tls : 0.f;
         loss[n] = -(tl - log_sum);
         // the row's base-2 normaliser, from which dlogits can be formed
         // elsewhere with the same bits (ce_dlogit8)
@@ -206,6 +208,7 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
     }
     if (!dlogits) return;
     bf16x8v* dL = (bf16x8v*)(dlogits + n * (int64_t)V);
+    const int tc = hit ? tgt >> 3 : -1;  // the chunk that holds the target
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
         const int c = threadIdx.x + 1024 * k;
@@ -213,10 +216,14 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
             float f[8];
             unpack8(r[k], f);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(f[e], kLog2e, -ls2));
-                f[e] = (p - (float)(c * 8 + e == tgt)) * inv_N;
+            for (int e = 0; e < 8; e++)
+                f[e] = __builtin_amdgcn_exp2f(fmaf(f[e], kLog2e, -ls2));
+            if (c == tc) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) f[e] -= (float)(e == (tgt & 7));
             }
+#pragma unroll
+            for (int e = 0; e < 8; e++) f[e] *= inv_N;
             dL[c] = pack8(f);
         }
     }
