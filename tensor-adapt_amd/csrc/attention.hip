@@ -243,7 +243,11 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16* __restrict__ Q,
     const float sl2 = scale * kLog2e;
     Rows64<HD> lk, lv;
 
-    // pass 1: online max / sum of exp2 (per-lane partial sums, shared max)
+    // pass 1: online max / sum of exp2, per lane over its own keys (16 lanes
+    // share a row); the lanes combine once after the last tile.  A shared
+    // running max would put two 4-step cross-lane exchanges per row on every
+    // tile's critical path, which bounds this kernel: at 4 x 512 tokens every
+    // block is resident and the longest walks 8 tiles twice.
     float m[4], l[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -269,11 +273,13 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16* __restrict__ Q,
                 v[t] = (!diag || (key <= row && key < T)) ? S[t][r] * sl2 : -INFINITY;
                 tmax = fmaxf(tmax, v[t]);
             }
-            const float mn = fmaxf(m[r], red16_max(tmax));
+            const float mn = fmaxf(m[r], tmax);
+            // (a lane without a key of this row so far: exponents of -inf)
+            const float ms = mn == -INFINITY ? 0.f : mn;
             float add = 0.f;
 #pragma unroll
-            for (int t = 0; t < 4; t++) add += exp2_fast(v[t] - mn);
-            l[r] = (m[r] == -INFINITY ? 0.f : l[r] * exp2_fast(m[r] - mn)) + add;
+            for (int t = 0; t < 4; t++) add += exp2_fast(v[t] - ms);
+            l[r] = l[r] * exp2_fast(m[r] - ms) + add;
             m[r] = mn;
         }
     }
@@ -281,7 +287,9 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16* __restrict__ Q,
     bool rowok[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        inv[r] = 1.f / red16_sum(l[r]);
+        const float mr = red16_max(m[r]);  // finite: key 0 precedes every row
+        inv[r] = 1.f / red16_sum(l[r] * exp2_fast(m[r] - mr));
+        m[r] = mr;
         rowok[r] = rbase + r < T;
         // (max, 1 / sum) of the row: P = exp2(S scale log2e - max) / sum is
         // recomputed from them, bit for bit, where P is not stored
@@ -349,13 +357,16 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16* __restrict__ Q,
     }
     // zeros above the diagonal (ops.cu:352-396 leaves exact zeros there)
     if (SP && zero_fill) {
-        int k0 = (qt + 1) * TK;
-        int width = T - k0;
-        if (width > 0) {
-            for (int i = threadIdx.x; i < TQ * width; i += 256) {
-                int r = i / width, c = i % width;
-                if (q0 + r < T) Ph[(int64_t)(q0 + r) * T + k0 + c] = 0.f;
-            }
+        // a wave takes whole rows; 16-byte stores where rows keep that alignment
+        const int k0 = (qt + 1) * TK;
+        const bool v4 = (T & 3) == 0 && ((uintptr_t)Ph & 15u) == 0;
+        for (int r = w; r < TQ && q0 + r < T; r += 4) {
+            float* row = Ph + (int64_t)(q0 + r) * T;
+            if (v4)
+                for (int c = k0 + 4 * lane; c < T; c += 256)
+                    *(float4*)(row + c) = make_float4(0.f, 0.f, 0.f, 0.f);
+            else
+                for (int c = k0 + lane; c < T; c += 64) row[c] = 0.f;
         }
     }
     // O (bf16, and F32 when O32 is given) — lane holds column 16j + l%16 of
@@ -1290,8 +1301,25 @@ __global__ __launch_bounds__(256) void k_attn_rowdot_o(const bf16* __restrict__ 
     }
 }
 
+// P values a lane needs for one key tile in the C layout of a 16 x 64 wave
+// tile: p[t][r] = P[row0 + r][key0 + 16t + l%16] for keys <= row (0 above).
+__device__ __forceinline__ void load_p_rows(float (&p)[4][4], const float* __restrict__ Ph, int T,
+                                            int row0, int key0, int lane) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        int key = key0 + 16 * t + (lane & 15);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            int row = row0 + r;
+            p[t][r] = (key <= row && key < T && row < T) ? Ph[(int64_t)row * T + key] : 0.f;
+        }
+    }
+}
+
 // Without the F32 output (the C-ABI's sdpa_bwd): D = sum_k P * dP with
-// dP = dO V^T recomputed on MFMA, per (b, hq, query tile).
+// dP = dO V^T recomputed on MFMA, per (b, hq, query tile).  The next tile's V
+// and P are loaded while the current one computes: P is most of the bytes,
+// and loading it where it is used put its latency on every tile.
 template <int HD>
 __global__ __launch_bounds__(256) void k_attn_rowdot_p(const bf16* __restrict__ dO,
                                                        const bf16* __restrict__ V,
@@ -1318,45 +1346,38 @@ __global__ __launch_bounds__(256) void k_attn_rowdot_p(const bf16* __restrict__ 
     int rbase = q0 + 16 * w + 4 * (lane >> 4);
     float dsum[4] = {0.f, 0.f, 0.f, 0.f};
     Rows64<HD> lv;
+    float pn[4][4];
     lv.load(Vh, ks_, 0, T);
+    load_p_rows(pn, Ph, T, rbase, 0, lane);
     for (int kt = 0; kt <= qt; kt++) {
         __syncthreads();
         lv.store(sV);
+        float pc[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) pc[t][r] = pn[t][r];
         __syncthreads();
-        if (kt < qt) lv.load(Vh, ks_, (kt + 1) * TK, T);
+        if (kt < qt) {
+            lv.load(Vh, ks_, (kt + 1) * TK, T);
+            load_p_rows(pn, Ph, T, rbase, (kt + 1) * TK, lane);
+        }
         floatx4 dP[4];
         wave_qk<HD>(dP, of, sV, lane);
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            int key = kt * TK + 16 * t + (lane & 15);
+        for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                int row = rbase + r;
-                if (key <= row && key < T && row < T)
-                    dsum[r] += Ph[(int64_t)row * T + key] * dP[t][r];
+                // (a key past the row takes no part, whatever its dP)
+                const int key = kt * TK + 16 * t + (lane & 15);
+                if (kt < qt || key <= rbase + r) dsum[r] += pc[t][r] * dP[t][r];
             }
-        }
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         float d = red16_sum(dsum[r]);
         int row = rbase + r;
         if ((lane & 15) == 0 && row < T) Dout[(int64_t)bh * T + row] = d;
-    }
-}
-
-// P values a lane needs for one key tile in the C layout of a 16 x 64 wave
-// tile: p[t][r] = P[row0 + r][key0 + 16t + l%16] for keys <= row (0 above).
-__device__ __forceinline__ void load_p_rows(float (&p)[4][4], const float* __restrict__ Ph, int T,
-                                            int row0, int key0, int lane) {
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        int key = key0 + 16 * t + (lane & 15);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            int row = row0 + r;
-            p[t][r] = (key <= row && key < T && row < T) ? Ph[(int64_t)row * T + key] : 0.f;
-        }
     }
 }
 
