@@ -227,7 +227,8 @@ int ta_centroid_accumulate_f32n(const float* h, const float* n, int64_t BT, int 
  * replaces the Lloyd loop of CentroidAccumulator::merge_and_write
  * src/centroid/centroid_accumulator.cpp:114-157: init center i =
  * snaps[(i*N)/k], <= max_iters iterations, strict-< ties, stop when no
- * assignment changes, empty cluster -> zero vector.  One device launch.
+ * assignment changes, empty cluster -> zero vector.  Launches only, no host
+ * synchronisation.
  * k is clamped to N (centers then holds min(k, N) rows); iters_out (device
  * int, may be NULL) receives the number of assignment passes that changed
  * something, as the reference's loop counter. */

@@ -417,7 +417,6 @@ __device__ __forceinline__ void kmeans_update(const float* __restrict__ X, int s
 // Snapshots that fit kXs floats are copied into LDS once (XL, permuted as
 // above): the distance chains and the center sums then read them from LDS.
 constexpr int kXs = 32768;  // 128 KB
-constexpr int kDs = 4096;   // distances held in LDS by k_kmeans_pp<true>
 
 template <bool XL>
 __device__ __forceinline__ const float* stage_snapshots(const float* __restrict__ Xg, float* xs,
@@ -460,169 +459,434 @@ __global__ __launch_bounds__(1024) void k_kmeans_ref(const float* __restrict__ X
     if (threadIdx.x == 0 && iters_out) *iters_out = it;
 }
 
-// Phases of k_kmeans_pp: the whole merge in one launch, or (the Lloyd
-// iterations spread over many workgroups in launches of their own,
-// k_kmeans_dist + k_kmeans_step) the seeding up to the initial centers and
-// zero assignments, and the ranking after the last assignment.
-enum KmPhase { KM_ALL = 0, KM_SEED = 1, KM_RANK = 2 };
+// ── k-means spread over the GPU ───────────────────────────────────────────
+// Every value is a chain of F32 (or F64) additions that has to run in order,
+// so what the work costs is latency: the chains of a pass run side by side,
+// one per lane, and a Lloyd iteration is one launch of one block per center
+// (k_kmeans_iter) with nothing to wait for inside a launch.  The snapshots
+// are kept transposed as well, so that 64 chains read 64 neighbouring values.
+// 64 snapshots of 512, k = 32, 25 passes: 139 us, against 844 us with the
+// distances spread out and everything else on one workgroup, and 3.1 ms on
+// one workgroup alone.
 
-template <bool XL, int PH = KM_ALL>
-__global__ __launch_bounds__(1024) void k_kmeans_pp(const float* __restrict__ Xg,
-                                                    const float* __restrict__ W, int N, int D,
-                                                    int k, int iters, uint64_t seed,
-                                                    float* __restrict__ Cw,  // [k*D] work
-                                                    float* __restrict__ d2g,  // [N]
-                                                    float* __restrict__ distg,  // [k*N]
-                                                    int32_t* __restrict__ asgg,  // [N]
-                                                    int32_t* __restrict__ chosen_g,  // [k]
-                                                    float* __restrict__ C_out,
-                                                    int32_t* __restrict__ asg_out,
-                                                    double* __restrict__ mass_out,
-                                                    int32_t* __restrict__ seeds_out, bool vec) {
-    // XL (N*D <= kXs, N <= 1024, N*k <= kDs): snapshots, assignments,
-    // distances and the seeding distances in LDS; the ranking arrays reuse
-    // the snapshot region once the last assignment pass has read it
-    __shared__ int chosen[1024];
-    __shared__ uint64_t rng;
-    __shared__ __attribute__((aligned(16))) float xs[XL ? kXs : 1];
-    __shared__ int sasg[XL ? 1024 : 1];
-    __shared__ float sdist[XL ? kDs : 1];
-    __shared__ float sd2[XL ? 1024 : 1];
-    __shared__ double smass[XL ? 1 : 1024];
-    __shared__ int sorder[XL ? 1 : 1024], srank[XL ? 1 : 1024];
-    int sw = 0;
-    const float* __restrict__ X =
-        PH == KM_RANK ? Xg : stage_snapshots<XL>(Xg, xs, N, D, sw);
-    // (the split phases keep the assignments in global memory)
-    int32_t* asg = XL && PH == KM_ALL ? sasg : asgg;
-    float* dist = XL ? sdist : distg;
-    float* d2 = XL ? sd2 : d2g;
-    double* mass = XL ? (double*)xs : smass;
-    int* order = XL ? (int*)(xs + 2 * 1024) : sorder;
-    int* rank_of = XL ? (int*)(xs + 3 * 1024) : srank;
-    if constexpr (PH != KM_RANK) {
-    if (threadIdx.x == 0) {
-        rng = seed;
+// values of a center or snapshot held in LDS; k_kmeans_cdist forms the
+// distances of longer centers
+constexpr int kIterC = 4096;
+
+// XT[d][n] = X[n][d], 32 x 32 tiles
+__global__ __launch_bounds__(256) void k_kmeans_transpose(const float* __restrict__ X,
+                                                          float* __restrict__ XT, int N, int D) {
+    __shared__ float t[32][33];
+    const int n0 = blockIdx.x * 32, d0 = blockIdx.y * 32, c = threadIdx.x & 31;
+    for (int r = threadIdx.x >> 5; r < 32; r += 8)
+        if (n0 + r < N && d0 + c < D) t[r][c] = X[(int64_t)(n0 + r) * D + d0 + c];
+    __syncthreads();
+    for (int r = threadIdx.x >> 5; r < 32; r += 8)
+        if (d0 + r < D && n0 + c < N) XT[(int64_t)(d0 + r) * N + n0 + c] = t[c][r];
+}
+
+// The chain of snapshot n (column n of XT) against the D values at b (read
+// at one address by all lanes).  32 elements at a time: the next 32 are in
+// flight, the squares form independently of one another, and only the
+// additions wait for each other.
+__device__ __forceinline__ void col32(const float* __restrict__ XT, int N, uint32_t n, int i,
+                                      float (&v)[32]) {
+#pragma unroll
+    for (int u = 0; u < 32; u++) v[u] = (XT + (int64_t)(i + u) * N)[n];
+}
+__device__ __forceinline__ float chain32(float d, const float (&v)[32], const float* b) {
+    float q[32];
+#pragma unroll
+    for (int u = 0; u < 32; u++) q[u] = b[u];
+#pragma unroll
+    for (int u = 0; u < 32; u++) q[u] = sq_term(v[u], q[u]);
+#pragma unroll
+    for (int u = 0; u < 32; u++) d = __fadd_rn(d, q[u]);
+    return d;
+}
+__device__ __forceinline__ float sqdist_col(const float* __restrict__ XT, int N, int D, uint32_t n,
+                                            const float* b) {
+    float d = 0.f;
+    int i = 0;
+    if (D >= 32) {
+        float v[32], w[32];
+        col32(XT, N, n, 0, v);
+        for (; i + 96 <= D; i += 64) {
+            col32(XT, N, n, i + 32, w);
+            d = chain32(d, v, b + i);
+            col32(XT, N, n, i + 64, v);
+            d = chain32(d, w, b + i + 32);
+        }
+        if (i + 64 <= D) {
+            col32(XT, N, n, i + 32, w);
+            d = chain32(d, v, b + i);
+            d = chain32(d, w, b + i + 32);
+            i += 64;
+        } else {
+            d = chain32(d, v, b + i);
+            i += 32;
+        }
+    }
+    for (; i < D; i++) d = __fadd_rn(d, sq_term((XT + (int64_t)i * N)[n], b[i]));
+    return d;
+}
+
+// out[r][n]: distance of snapshot n to snapshot r (block x = r, 64 snapshots
+// per block), or, with k > 0, to the r-th of the reference's k initial
+// centers, snapshot (r N) / k, which is also copied to C[r]
+__global__ __launch_bounds__(64) void k_kmeans_rows(const float* __restrict__ X,
+                                                    const float* __restrict__ XT, int N, int D,
+                                                    int k, float* __restrict__ C,
+                                                    float* __restrict__ out,
+                                                    int32_t* __restrict__ done) {
+    __shared__ __attribute__((aligned(16))) float b[kIterC];
+    const int r = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
+    const int row = k > 0 ? (int)(((int64_t)r * N) / k) : r;
+    if (D <= kIterC) {
+        for (int i = threadIdx.x; i < D; i += 64) b[i] = X[(int64_t)row * D + i];
+        __syncthreads();
+    }
+    const float d = D <= kIterC ? sqdist_col(XT, N, D, min(n, N - 1), b)
+                                : sqdist_col(XT, N, D, min(n, N - 1), X + (int64_t)row * D);
+    if (n < N) out[(int64_t)r * N + n] = d;
+    if (k > 0 && blockIdx.y == 0) {
+        for (int i = threadIdx.x; i < D; i += 64) C[(int64_t)r * D + i] = X[(int64_t)row * D + i];
+        if (r == 0 && threadIdx.x == 0) *done = 0;
+    }
+}
+
+// k-means++ seeding (one block), then the initial centers C and their
+// distances dist [k][N].  A draw's running sum is an F64 chain in index
+// order, kept per snapshot (pre), so the pick is the first snapshot whose
+// prefix passes the target.
+//
+// PD: the distances between all snapshots [N][N] (N <= 1024).  Wave 0 then
+// draws alone, from rows of PD (in LDS for N <= 128), with nothing to wait
+// for but its own chain: 31 draws over 64 snapshots took 128 us with the
+// block's barriers and a row from global memory in each.  PD NULL: the block
+// forms each draw's chains to the center drawn last.
+constexpr int kPairMax = 1024, kPairLds = 128;
+__global__ __launch_bounds__(1024) void k_kmeans_seed(const float* __restrict__ X,
+                                                      const float* __restrict__ XT,
+                                                      const float* __restrict__ PD, int N, int D,
+                                                      int k, uint64_t seed, float* d2, double* pre,
+                                                      float* __restrict__ C,
+                                                      float* __restrict__ dist,
+                                                      int32_t* __restrict__ chosen,
+                                                      int32_t* __restrict__ done) {
+    __shared__ int last;
+    __shared__ float spd[kPairLds * kPairLds];
+    __shared__ float sd2[kPairMax];
+    __shared__ double spre[kPairMax];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const bool lds = PD && N <= kPairLds;
+    if (PD) {
+        d2 = sd2;
+        pre = spre;
+    }
+    if (lds)
+        for (int p = threadIdx.x; p < N * N; p += 1024) spd[p] = PD[p];
+    uint64_t rng = seed;  // wave 0's, the same in every lane
+    if (w == 0) {
         int first = (int)(u01(rng) * N);
         if (first >= N) first = N - 1;
-        chosen[0] = first;
+        if (lane == 0) {
+            chosen[0] = last = first;
+            *done = 0;
+        }
     }
-    for (int n = threadIdx.x; n < N; n += blockDim.x) d2[n] = FLT_MAX;
+    for (int n = threadIdx.x; n < N; n += 1024) d2[n] = FLT_MAX;
     __syncthreads();
-    // k-means++ seeding
-    for (int m = 1; m < k; m++) {
-        const int cm = chosen[m - 1];
-        for (int n = threadIdx.x; n < N; n += blockDim.x) {
-            const int nn[1] = {n};
-            const float* const cb[1] = {X + (int64_t)cm * D};
-            const int kb[1] = {cm & sw};
-            float d[1];
-            sqdist_chains<1, 32>(X, D, sw, vec, nn, cb, kb, d);
-            if (d[0] < d2[n]) d2[n] = d[0];
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double total = 0.0;
-            for (int n = 0; n < N; n++) total += (double)d2[n];
-            double target = u01(rng) * total;
-            int pick = -1, last_pos = -1;
-            double run = 0.0;
-            for (int n = 0; n < N; n++) {
-                run += (double)d2[n];
-                if (d2[n] > 0.f) last_pos = n;
-                if (pick < 0 && run > target && d2[n] > 0.f) pick = n;
+    // draw m by wave 0, from d2
+    auto draw = [&](int m) -> int {
+        double run = 0.0;
+        for (int n0 = 0; n0 < N; n0 += 64) {
+            const float v = n0 + lane < N ? d2[n0 + lane] : 0.f;
+            double mine = 0.0;
+            if (n0 + 64 <= N) {
+#pragma unroll
+                for (int l = 0; l < 64; l++) {
+                    run += (double)__uint_as_float(
+                        __builtin_amdgcn_readlane(__float_as_uint(v), l));
+                    mine = lane == l ? run : mine;
+                }
+            } else {
+                for (int l = 0; n0 + l < N; l++) {
+                    run += (double)__uint_as_float(
+                        __builtin_amdgcn_readlane(__float_as_uint(v), l));
+                    mine = lane == l ? run : mine;
+                }
             }
-            if (pick < 0) pick = (last_pos >= 0) ? last_pos : m % N;
-            chosen[m] = pick;
+            if (n0 + lane < N) pre[n0 + lane] = mine;
+        }
+        const double target = u01(rng) * run;
+        int pick = -1, last_pos = -1;
+        for (int n0 = 0; n0 < N; n0 += 64) {
+            const int n = n0 + lane;
+            const bool pos = n < N && d2[n] > 0.f;
+            const uint64_t some = __ballot(pos);
+            const uint64_t past = __ballot(pos && pre[n] > target);
+            if (some) last_pos = n0 + 63 - __builtin_clzll(some);
+            if (pick < 0 && past) pick = n0 + __builtin_ctzll(past);
+        }
+        return pick >= 0 ? pick : last_pos >= 0 ? last_pos : m % N;
+    };
+    if (PD) {
+        if (w == 0) {
+            int cm = __builtin_amdgcn_readfirstlane(last);
+            for (int m = 1; m < k; m++) {
+                // (one wave: each lane reads back only what it wrote itself)
+                for (int n = lane; n < N; n += 64) {
+                    const float d = lds ? spd[cm * N + n] : PD[(int64_t)cm * N + n];
+                    if (d < d2[n]) d2[n] = d;
+                }
+                cm = draw(m);
+                if (lane == 0) chosen[m] = cm;
+            }
+        }
+    } else {
+        for (int m = 1; m < k; m++) {
+            const int cm = last;
+            for (int n = threadIdx.x; n < N; n += 1024) {
+                const float d = sqdist_col(XT, N, D, n, X + (int64_t)cm * D);
+                if (d < d2[n]) d2[n] = d;
+            }
+            __syncthreads();
+            if (w == 0) {
+                const int pick = draw(m);
+                if (lane == 0) chosen[m] = last = pick;
+            }
+            __syncthreads();
+        }
+    }
+    __syncthreads();
+    for (int c = w; c < k; c += 16) {
+        const int row = chosen[c];
+        for (int i = lane; i < D; i += 64) C[(int64_t)c * D + i] = X[(int64_t)row * D + i];
+        for (int n = lane; n < N; n += 64)
+            dist[(int64_t)c * N + n] = PD ? PD[(int64_t)row * N + n]
+                                          : sqdist_col(XT, N, D, n, X + (int64_t)row * D);
+    }
+}
+
+// The nearest center (strict <, so the first of equal distances; 0 when none
+// is below 1e38) of snapshots n0 .. n0 + 63, one per lane, from dist [k][N]:
+// the block's four waves take a quarter of the centers each and wave 0 joins
+// them in center order.  The result is valid in wave 0; the caller puts a
+// barrier between calls.
+__device__ __forceinline__ int nearest64(const float* __restrict__ dist, int N, int k, int n0,
+                                         float (&sb)[4][64], int (&si)[4][64]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, kq = (k + 3) / 4;
+    const int n = min(n0 + lane, N - 1), c1 = min(k, (w + 1) * kq);
+    float best = 1e38f;
+    int bk = 0;
+    for (int c0 = w * kq; c0 < c1; c0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = c0 + u < c1 ? dist[(int64_t)(c0 + u) * N + n] : 1e38f;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (c0 + u < c1 && v[u] < best) {
+                best = v[u];
+                bk = c0 + u;
+            }
+    }
+    sb[w][lane] = best;
+    si[w][lane] = bk;
+    __syncthreads();
+    best = 1e38f;
+    bk = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (sb[q][lane] < best) {
+            best = sb[q][lane];
+            bk = si[q][lane];
+        }
+    return bk;
+}
+
+// Iteration `it` of Lloyd's loop, block c for center c: every snapshot's
+// nearest center from the distances din [k][N] (each block for itself: N x k
+// loads), center c as the mean of its members summed in snapshot index order,
+// and the new center's distances into dout.  An empty center becomes zero
+// (REF, the reference's loop) or stays.  A pass that changes no assignment
+// ends the loop: the centers and distances of every later pass would be the
+// same values, so *done makes later launches return at once.  (A block of
+// the same launch that sees it early skips what is unchanged anyway.)
+// asg_in / asg_out: the previous and this pass's assignments (REF's first
+// pass compares against zeros); asg_fin always holds the latest.
+template <bool REF>
+__global__ __launch_bounds__(256) void k_kmeans_iter(
+    const float* __restrict__ X, const float* __restrict__ XT, float* __restrict__ C, int N, int D,
+    int k, int it, const float* __restrict__ din, float* __restrict__ dout,
+    const int32_t* __restrict__ asg_in, int32_t* __restrict__ asg_out,
+    int32_t* __restrict__ asg_fin, uint64_t* __restrict__ masks, int32_t* done,
+    int32_t* __restrict__ iters_out, bool last) {
+    __shared__ float sb[4][64];
+    __shared__ int si[4][64];
+    __shared__ __attribute__((aligned(16))) float cen[kIterC];
+    __shared__ uint64_t smask[64];
+    if (*(volatile int32_t*)done) return;
+    const int c = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nb = (N + 63) / 64;
+    // members of c, a bit per snapshot (in LDS up to 4096 snapshots)
+    uint64_t* const mask = nb <= 64 ? smask : masks + (int64_t)c * nb;
+    int changed = !REF && it == 0;
+    for (int j = 0; j < nb; j++) {
+        const int n = 64 * j + lane;
+        const int a = nearest64(din, N, k, 64 * j, sb, si);
+        if (w == 0) {
+            const uint64_t mem = __ballot(n < N && a == c);
+            if (lane == 0) mask[j] = mem;
+            if (n < N) {
+                if (it > 0 || REF) changed |= (it == 0 ? 0 : asg_in[n]) != a;
+                if (c == 0) asg_out[n] = asg_fin[n] = a;
+            }
         }
         __syncthreads();
     }
-    for (int p = threadIdx.x; p < k * D; p += blockDim.x) {
-        const int n = chosen[p / D], d = p % D;
-        Cw[p] = X[(int64_t)n * D + snap_col(n, d, sw)];
-    }
-    for (int n = threadIdx.x; n < N; n += blockDim.x) asg[n] = 0;
-    if constexpr (PH == KM_SEED) {
-        for (int r = threadIdx.x; r < k; r += blockDim.x) chosen_g[r] = chosen[r];
+    changed = __syncthreads_or(changed);
+    if (!changed) {
+        if (c == 0 && threadIdx.x == 0) {
+            if (REF && iters_out) *iters_out = it;
+            *done = 1;
+        }
         return;
     }
-    __syncthreads();
-    for (int it = 0; it < iters; it++) {
-        kmeans_assign(X, sw, vec, Cw, N, D, k, dist, asg);
-        kmeans_update(X, sw, Cw, N, D, k, asg, false);
+    if (REF && c == 0 && threadIdx.x == 0 && iters_out) *iters_out = it + 1;
+    float* const Cc = C + (int64_t)c * D;
+    const bool with_dist = !last && D <= kIterC;
+    for (int d = threadIdx.x; d < D; d += 256) {
+        float s = 0.f;
+        int cnt = 0;
+        for (int j = 0; j < nb; j++) {
+            uint64_t mem = mask[j];
+            cnt += __popcll(mem);
+            // up to eight members' values loaded together, added in order
+            while (mem) {
+                float xv[8];
+                int nm = 0;
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    if (!mem) break;
+                    xv[u] = X[(int64_t)(64 * j + __builtin_ctzll(mem)) * D + d];
+                    mem &= mem - 1;
+                    nm++;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (u < nm) s = __fadd_rn(s, xv[u]);
+            }
+        }
+        const float v = cnt > 0 ? s / (float)cnt : REF ? 0.f : Cc[d];
+        Cc[d] = v;
+        if (with_dist) cen[d] = v;
     }
-    kmeans_assign(X, sw, vec, Cw, N, D, k, dist, asg);
-    } else {
-        for (int r = threadIdx.x; r < k; r += blockDim.x) chosen[r] = chosen_g[r];
+    if (!with_dist) return;
+    __syncthreads();
+    for (int j = w; j < nb; j += 4) {
+        const int n = 64 * j + lane;
+        const float d = sqdist_col(XT, N, D, min(n, N - 1), cen);
+        if (n < N) dout[(int64_t)c * N + n] = d;
+    }
+}
+
+// dist[c][n] of centers too long for k_kmeans_iter's LDS (blocks of 64
+// snapshots), after its launch
+__global__ __launch_bounds__(64) void k_kmeans_cdist(const float* __restrict__ XT,
+                                                     const float* __restrict__ C, int N, int D,
+                                                     float* __restrict__ dist,
+                                                     const int32_t* __restrict__ done) {
+    if (*done) return;
+    const int c = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
+    const float d = sqdist_col(XT, N, D, min(n, N - 1), C + (int64_t)c * D);
+    if (n < N) dist[(int64_t)c * N + n] = d;
+}
+
+// Final assignments (from the last distances unless the loop ended on a
+// fixed point), then the centers ranked by the weight of their members:
+// masses summed in F64 in snapshot index order, one lane per center; stable
+// descending order (a center's rank is the number of centers that precede
+// it; with a NaN mass, which no count can order, the insertion sort that
+// defines the order runs as it stands).
+__global__ __launch_bounds__(1024) void k_kmeans_rank(const float* __restrict__ W, int N, int D,
+                                                      int k, const float* __restrict__ dist,
+                                                      const float* __restrict__ C,
+                                                      int32_t* __restrict__ asg,
+                                                      const int32_t* __restrict__ chosen,
+                                                      const int32_t* __restrict__ done,
+                                                      float* __restrict__ C_out,
+                                                      int32_t* __restrict__ asg_out,
+                                                      double* __restrict__ mass_out,
+                                                      int32_t* __restrict__ seeds_out) {
+    __shared__ double mass[1024];
+    __shared__ int order[1024], rank_of[1024];
+    __shared__ float sw[1024];
+    __shared__ int sa[1024];
+    const int t = threadIdx.x;
+    const bool have = *done != 0;
+    double m = 0.0;
+    for (int n0 = 0; n0 < N; n0 += 1024) {
+        const int n = n0 + t, cnt = min(1024, N - n0);
+        if (n < N) {
+            int bk = 0;
+            if (have) {
+                bk = asg[n];
+            } else {
+                float best = 1e38f;
+                for (int c0 = 0; c0 < k; c0 += 16) {
+                    float v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; u++)
+                        v[u] = c0 + u < k ? dist[(int64_t)(c0 + u) * N + n] : 1e38f;
+#pragma unroll
+                    for (int u = 0; u < 16; u++)
+                        if (c0 + u < k && v[u] < best) {
+                            best = v[u];
+                            bk = c0 + u;
+                        }
+                }
+                asg[n] = bk;
+            }
+            sa[t] = bk;
+            sw[t] = W[n];
+        }
+        __syncthreads();
+        if (t < k)
+            for (int i = 0; i < cnt; i++)
+                if (sa[i] == t) m += (double)sw[i];
         __syncthreads();
     }
-    // rank by member weight (F64, index order), stable descending
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < k; c++) mass[c] = 0.0;
-        for (int n = 0; n < N; n++) mass[asg[n]] += (double)W[n];
-        for (int c = 0; c < k; c++) order[c] = c;
-        for (int i = 1; i < k; i++) {  // insertion sort: stable
-            int v = order[i];
-            int j = i - 1;
-            while (j >= 0 && mass[order[j]] < mass[v]) {
-                order[j + 1] = order[j];
-                j--;
-            }
-            order[j + 1] = v;
-        }
-        for (int r = 0; r < k; r++) rank_of[order[r]] = r;
-    }
-    __syncthreads();
-    for (int p = threadIdx.x; p < k * D; p += blockDim.x)
-        C_out[p] = Cw[(int64_t)order[p / D] * D + (p % D)];
-    for (int n = threadIdx.x; n < N; n += blockDim.x) asg_out[n] = rank_of[asg[n]];
-    for (int r = threadIdx.x; r < k; r += blockDim.x) {
-        if (mass_out) mass_out[r] = mass[order[r]];
-        if (seeds_out) seeds_out[r] = chosen[r];
-    }
-}
-
-// One Lloyd assignment pass spread over the GPU: block (c, j) is one wave
-// with center c against snapshots 64 j .. 64 j + 63 (one distance chain per
-// lane, the order of sqdist_chains), into dist [k][N].
-__global__ __launch_bounds__(64) void k_kmeans_dist(const float* __restrict__ X,
-                                                    const float* __restrict__ C, int N, int D,
-                                                    bool vec, float* __restrict__ dist) {
-    const int c = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
-    const int nn[1] = {min(n, N - 1)};
-    const float* const cb[1] = {C + (int64_t)c * D};
-    const int kb[1] = {0};
-    float d[1];
-    sqdist_chains<1, 64>(X, D, 0, vec, nn, cb, kb, d);
-    if (n < N) dist[(int64_t)c * N + n] = d[0];
-}
-
-// Then each snapshot's argmin over dist (strict <, as kmeans_assign) and,
-// with update, the centers' member means (kmeans_update, stress mode).
-__global__ __launch_bounds__(1024) void k_kmeans_step(const float* __restrict__ X,
-                                                      float* __restrict__ C, int N, int D, int k,
-                                                      const float* __restrict__ dist,
-                                                      int32_t* __restrict__ asg, bool update) {
-    for (int n = threadIdx.x; n < N; n += blockDim.x) {
-        // (the distances come from global memory: 16 loads in flight)
-        float best = 1e38f;
-        int bk = 0;
-        for (int c0 = 0; c0 < k; c0 += 16) {
-            float v[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) v[u] = c0 + u < k ? dist[(int64_t)(c0 + u) * N + n] : 0.f;
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (c0 + u < k && v[u] < best) {
-                    best = v[u];
-                    bk = c0 + u;
+    if (t < k) mass[t] = m;
+    if (__syncthreads_or(t < k && m != m)) {
+        if (t == 0) {
+            for (int c = 0; c < k; c++) order[c] = c;
+            for (int i = 1; i < k; i++) {  // insertion sort: stable
+                const int v = order[i];
+                int j = i - 1;
+                while (j >= 0 && mass[order[j]] < mass[v]) {
+                    order[j + 1] = order[j];
+                    j--;
                 }
+                order[j + 1] = v;
+            }
+            for (int r = 0; r < k; r++) rank_of[order[r]] = r;
         }
-        asg[n] = bk;
+    } else if (t < k) {
+        int r = 0;
+        for (int j = 0; j < k; j++) r += mass[j] > m || (mass[j] == m && j < t);
+        rank_of[t] = r;
+        order[r] = t;
     }
-    if (!update) return;
     __syncthreads();
-    kmeans_update(X, 0, C, N, D, k, asg, false);
+    for (int r = t >> 6; r < k; r += 16)
+        for (int i = t & 63; i < D; i += 64)
+            C_out[(int64_t)r * D + i] = C[(int64_t)order[r] * D + i];
+    for (int n = t; n < N; n += 1024) asg_out[n] = rank_of[asg[n]];
+    if (t < k) {
+        if (mass_out) mass_out[t] = mass[order[t]];
+        if (seeds_out) seeds_out[t] = chosen[t];
+    }
 }
 
 }  // namespace ta
@@ -686,6 +950,57 @@ struct DeviceScope {
     }
 };
 
+// Work arrays of the merge, carved from one scratch buffer.  pd_rows: rows of
+// the snapshot-to-snapshot distances (0: the reference's loop, which seeds
+// from fixed snapshots and keeps its centers and assignments in the caller's
+// arrays).
+struct KmeansScratch {
+    float *xt, *pd, *d2, *c, *dist[2];
+    double* pre;
+    uint64_t* masks;
+    int32_t *asg[3], *chosen, *done;
+    bool get(int N, int D, int k, int pd_rows, hipStream_t s) {
+        const bool pp = pd_rows > 0;
+        const int64_t nb = (N + 63) / 64;
+        const size_t n = (size_t)N, sz[] = {n * D * 4,
+                                            pp ? (size_t)pd_rows * N * 4 : 0,
+                                            pp ? n * 4 : 0,
+                                            pp ? (size_t)k * D * 4 : 0,
+                                            n * k * 4,
+                                            n * k * 4,
+                                            pp ? n * 8 : 0,
+                                            nb > 64 ? (size_t)k * nb * 8 : 0,
+                                            n * 4,
+                                            n * 4,
+                                            n * 4,
+                                            (size_t)k * 4,
+                                            4};
+        size_t off[13], total = 0;
+        for (int i = 0; i < 13; i++) {
+            off[i] = total;
+            total += (sz[i] + 255) & ~(size_t)255;
+        }
+        char* b = (char*)ta::scratch_get(total, s);
+        if (!b) return false;
+        xt = (float*)(b + off[0]);
+        pd = (float*)(b + off[1]);
+        d2 = (float*)(b + off[2]);
+        c = (float*)(b + off[3]);
+        dist[0] = (float*)(b + off[4]);
+        dist[1] = (float*)(b + off[5]);
+        pre = (double*)(b + off[6]);
+        masks = (uint64_t*)(b + off[7]);
+        for (int i = 0; i < 3; i++) asg[i] = (int32_t*)(b + off[8 + i]);
+        chosen = (int32_t*)(b + off[11]);
+        done = (int32_t*)(b + off[12]);
+        return true;
+    }
+};
+// Most passes the reference's loop launches one by one (its own cap is 50): a
+// launch after the last change still costs about 2 us, and beyond this the
+// loop on one workgroup, which stops by itself, is kept.
+constexpr int kRefLaunches = 128;
+
 extern "C" {
 
 int ta_centroid_accumulate_bf16(const uint16_t* h, const uint16_t* g, int64_t BT, int D,
@@ -744,6 +1059,30 @@ int ta_kmeans_ref(const float* snaps, int N, int D, int k, int max_iters, float*
                k);
     if (k > N) k = N;
     hipStream_t s = (hipStream_t)stream;
+    // one workgroup while its passes cost less than launches (about 10 us each
+    // that changes something, 2 us each after that, up to the cap): with the
+    // snapshots in its LDS (N D <= 32768) below k N D = 2^20 (64 x 512: k = 8
+    // 86 us against 102 with 25 passes launched, k = 32 127 against 96), read
+    // from global memory below 2^17 (32 x 1536, k = 2: 127 against 130; 96 x
+    // 512, k = 8: 373 against 99)
+    const bool small = (int64_t)k * N * D < (int64_t(1) << ((int64_t)N * D <= kXs ? 20 : 17));
+    if (!small && max_iters > 0 && max_iters <= kRefLaunches) {
+        KmeansScratch m;
+        TA_REQUIRE(m.get(N, D, k, 0, s), "kmeans_ref: scratch allocation failed");
+        tlaunch(k_kmeans_transpose, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), s, snaps, m.xt, N,
+                D);
+        tlaunch(k_kmeans_rows, dim3(k, (N + 63) / 64), dim3(64), s, snaps, m.xt, N, D, k, centers,
+                m.dist[0], m.done);
+        for (int it = 0; it < max_iters; it++) {
+            tlaunch(k_kmeans_iter<true>, dim3(k), dim3(256), s, snaps, m.xt, centers, N, D, k, it,
+                    m.dist[it & 1], m.dist[(it + 1) & 1], m.asg[it & 1], m.asg[(it + 1) & 1],
+                    assign, m.masks, m.done, iters_out, it + 1 == max_iters);
+            if (D > kIterC && it + 1 < max_iters)
+                tlaunch(k_kmeans_cdist, dim3(k, (N + 63) / 64), dim3(64), s, m.xt, centers, N, D,
+                        m.dist[(it + 1) & 1], m.done);
+        }
+        return check_launch("kmeans_ref");
+    }
     float* dist = (float*)scratch_get((size_t)N * k * sizeof(float), s);
     TA_REQUIRE(dist, "kmeans_ref: scratch allocation failed");
     // 16-byte operand loads: whole chunks, and aligned snapshots (when read
@@ -767,53 +1106,25 @@ int ta_kmeans_pp(const float* snaps, const float* weights, int N, int D, int k, 
     if (k > N) k = N;
     TA_REQUIRE(k <= 1024, "kmeans_pp: k=%d exceeds 1024", k);
     hipStream_t s = (hipStream_t)stream;
-    size_t off_d2 = (size_t)k * D * sizeof(float);
-    off_d2 = (off_d2 + 255) & ~(size_t)255;
-    size_t off_dist = off_d2 + (((size_t)N * sizeof(float) + 255) & ~(size_t)255);
-    size_t off_asg = off_dist + (((size_t)N * k * sizeof(float) + 255) & ~(size_t)255);
-    size_t off_ch = off_asg + (((size_t)N * sizeof(int32_t) + 255) & ~(size_t)255);
-    size_t total = off_ch + (size_t)k * sizeof(int32_t);
-    char* base = (char*)scratch_get(total, s);
-    TA_REQUIRE(base, "kmeans_pp: scratch allocation failed");
-    // (the work centers sit at the scratch's 256-byte aligned start)
-    const bool xl = (int64_t)N * D <= kXs && N <= 1024 && (int64_t)N * k <= kDs;
-    const bool vec = D % 4 == 0 && (xl || ((uintptr_t)snaps & 15) == 0);
-    float* Cw = (float*)base;
-    float* d2 = (float*)(base + off_d2);
-    float* dist = (float*)(base + off_dist);
-    int32_t* asg = (int32_t*)(base + off_asg);
-    int32_t* ch = (int32_t*)(base + off_ch);
-    // Lloyd iterations on one workgroup while their distance work is small
-    // (each assignment pass: k N D chain steps on one CU); above that, each
-    // pass in launches of its own: the distances over k x ceil(N / 64)
-    // waves, then the argmin and the center sums on one workgroup (the same
-    // arithmetic in the same order, so the same bits)
-    const bool spread = (int64_t)k * N * D >= (int64_t(1) << 19) && iters > 0;
-    if (!spread) {
-        if (xl)
-            tlaunch(k_kmeans_pp<true>, dim3(1), dim3(1024), s, snaps, weights, N, D, k, iters,
-                    seed, Cw, d2, dist, asg, ch, centers, assign, mass, seeds, vec);
-        else
-            tlaunch(k_kmeans_pp<false>, dim3(1), dim3(1024), s, snaps, weights, N, D, k, iters,
-                    seed, Cw, d2, dist, asg, ch, centers, assign, mass, seeds, vec);
-        return check_launch("kmeans_pp");
+    KmeansScratch m;
+    const bool pairs = N <= kPairMax;
+    TA_REQUIRE(m.get(N, D, k, pairs ? N : 1, s), "kmeans_pp: scratch allocation failed");
+    tlaunch(k_kmeans_transpose, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), s, snaps, m.xt, N, D);
+    if (pairs)
+        tlaunch(k_kmeans_rows, dim3(N, (N + 63) / 64), dim3(64), s, snaps, m.xt, N, D, 0, nullptr,
+                m.pd, nullptr);
+    tlaunch(k_kmeans_seed, dim3(1), dim3(1024), s, snaps, m.xt, pairs ? m.pd : nullptr, N, D, k,
+            seed, m.d2, m.pre, m.c, m.dist[0], m.chosen, m.done);
+    for (int it = 0; it < iters; it++) {
+        tlaunch(k_kmeans_iter<false>, dim3(k), dim3(256), s, snaps, m.xt, m.c, N, D, k, it,
+                m.dist[it & 1], m.dist[(it + 1) & 1], m.asg[it & 1], m.asg[(it + 1) & 1], m.asg[2],
+                m.masks, m.done, nullptr, false);
+        if (D > kIterC)
+            tlaunch(k_kmeans_cdist, dim3(k, (N + 63) / 64), dim3(64), s, m.xt, m.c, N, D,
+                    m.dist[(it + 1) & 1], m.done);
     }
-    if (xl)
-        tlaunch(k_kmeans_pp<true, KM_SEED>, dim3(1), dim3(1024), s, snaps, weights, N, D, k, iters,
-                seed, Cw, d2, dist, asg, ch, centers, assign, mass, seeds, vec);
-    else
-        tlaunch(k_kmeans_pp<false, KM_SEED>, dim3(1), dim3(1024), s, snaps, weights, N, D, k,
-                iters, seed, Cw, d2, dist, asg, ch, centers, assign, mass, seeds, vec);
-    // the passes read the snapshots from global memory: 16-byte loads need
-    // them aligned
-    const bool gvec = D % 4 == 0 && ((uintptr_t)snaps & 15) == 0;
-    const dim3 dgrid(k, (N + 63) / 64);
-    for (int it = 0; it <= iters; it++) {
-        tlaunch(k_kmeans_dist, dgrid, dim3(64), s, snaps, Cw, N, D, gvec, dist);
-        tlaunch(k_kmeans_step, dim3(1), dim3(1024), s, snaps, Cw, N, D, k, dist, asg, it < iters);
-    }
-    tlaunch(k_kmeans_pp<false, KM_RANK>, dim3(1), dim3(1024), s, snaps, weights, N, D, k, iters,
-            seed, Cw, d2, dist, asg, ch, centers, assign, mass, seeds, vec);
+    tlaunch(k_kmeans_rank, dim3(1), dim3(1024), s, weights, N, D, k, m.dist[iters & 1], m.c,
+            m.asg[2], m.chosen, m.done, centers, assign, mass, seeds);
     return check_launch("kmeans_pp");
 }
 

@@ -1,0 +1,98 @@
+"""The merge's launches (one block per center and Lloyd pass) at their edges,
+bit for bit against the oracle: around 64 snapshots per chunk, past 4096 (the
+member bits then leave LDS) and past 1024 (the seeding then forms its chains
+per draw), dimensions off and past the 32-element and LDS center sizes, data
+that settles at once and data that does not, duplicates (empty centers),
+few and many passes, and the one-workgroup loop beyond 128 passes."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from gpu_util import DEV, P, S, call, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def data(N, D, kind):
+    r = np.random.default_rng(N * 7 + D)
+    if kind == "mixture":
+        means = r.standard_normal((5, D))
+        X = means[r.integers(0, 5, N)] + 0.3 * r.standard_normal((N, D))
+    elif kind == "spread":
+        X = r.standard_normal((N, D))
+    else:  # three points, repeated: empty centers
+        X = r.standard_normal((3, D))[r.integers(0, 3, N)]
+    return np.ascontiguousarray(X.astype(np.float32)), r.lognormal(0, 1, N).astype(np.float32)
+
+
+SHAPES = [(1, 1, 1, 5), (2, 3, 2, 4), (63, 33, 9, 25), (64, 512, 32, 25), (65, 500, 32, 7),
+          (130, 31, 40, 25), (1030, 17, 6, 12), (4200, 5, 4, 6), (20, 4100, 5, 6)]
+
+
+@pytest.mark.parametrize("kind", ["mixture", "spread", "dups"])
+@pytest.mark.parametrize("N,D,k,iters", SHAPES)
+def test_pp(N, D, k, iters, kind):
+    X, W = data(N, D, kind)
+    C = torch.empty(k * D, device=DEV)
+    A = torch.empty(N, dtype=torch.int32, device=DEV)
+    M = torch.empty(k, dtype=torch.float64, device=DEV)
+    Sd = torch.empty(k, dtype=torch.int32, device=DEV)
+    call("ta_kmeans_pp", P(dev(X)), P(dev(W)), N, D, k, iters, ctypes.c_uint64(77), P(C), P(A),
+         P(M), P(Sd), S())
+    rc, ra, rm, rs = O.kmeans_pp(X, W, k, iters, 77)
+    assert np.array_equal(host(Sd), rs) and np.array_equal(host(A), ra)
+    assert np.array_equal(host(C).reshape(k, D), rc)
+    assert np.allclose(host(M), rm, rtol=1e-12)
+
+
+@pytest.mark.parametrize("kind", ["mixture", "spread", "dups"])
+@pytest.mark.parametrize("N,D,k,iters", SHAPES)
+def test_ref(N, D, k, iters, kind):
+    X, _ = data(N, D, kind)
+    out = []
+    for cap in (50, 200):  # one launch per pass; the one-workgroup loop
+        C = torch.empty(k * D, device=DEV)
+        A = torch.empty(N, dtype=torch.int32, device=DEV)
+        it = torch.empty(1, dtype=torch.int32, device=DEV)
+        call("ta_kmeans_ref", P(dev(X)), N, D, k, cap, P(C), P(A), P(it), S())
+        out.append((host(C).reshape(k, D), host(A), int(host(it)[0])))
+    rc, ra, ri = O.kmeans_ref(X, k)
+    for c, a, i in out[: 2 if out[1][2] <= 50 else 1]:
+        assert np.array_equal(a, ra) and np.array_equal(c, rc) and i == ri
+
+
+def test_few_passes_match_the_loop():
+    """A cap below the passes the data needs: centers after the last update,
+    assignments of the last pass; no pass at all leaves the initial centers."""
+    X, _ = data(90, 64, "spread")
+    for cap in (0, 1, 2, 3):
+        got = []
+        for big in (False, True):
+            C = torch.full((8 * 64,), -1.0, device=DEV)
+            A = torch.full((90,), -1, dtype=torch.int32, device=DEV)
+            it = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+            call("ta_kmeans_ref", P(dev(X)), 90, 64, 8, cap, P(C), P(A), P(it), S())
+            got.append((host(C), host(A), host(it)))
+        want_c = X[[(i * 90) // 8 for i in range(8)]].copy()
+        asg, n_it = np.zeros(90, np.int32), 0
+        for _ in range(cap):
+            d = np.zeros((90, 8), np.float32)
+            for i in range(64):
+                t = (X[:, None, i] - want_c[None, :, i]).astype(np.float32)
+                d = (d + (t * t).astype(np.float32)).astype(np.float32)
+            a = d.argmin(1).astype(np.int32)
+            if np.array_equal(a, asg):
+                break
+            asg, n_it = a, n_it + 1
+            for c in range(8):
+                mem = np.nonzero(asg == c)[0]
+                s = np.zeros(64, np.float32)
+                for n in mem:
+                    s = (s + X[n]).astype(np.float32)
+                want_c[c] = s / np.float32(len(mem)) if len(mem) else 0
+        for c, a, i in got:
+            assert np.array_equal(c.reshape(8, 64), want_c)
+            assert np.array_equal(a, asg) and int(i[0]) == n_it
