@@ -63,6 +63,12 @@ struct Engine {
     ta_model_config mc;
     ta_adapt_config ac;
     int B, T, BT, H, qd, kvd, I, V;
+    // BT rounded up to 64, the token tile of the fused LoRA backward kernels:
+    // what they read (the output gradients, gate, up and h) and write has that
+    // many rows, of which those past BT hold zeros and stay zero, so a batch of
+    // any length takes them (two 1.5B layers, 3 x 777 tokens: 4104 -> 4038 us a
+    // step against the per-pair kernels)
+    int BTp;
     // r: the rank every buffer and kernel of the engine is laid out for, the
     // requested rank r_real rounded up to a multiple of 16.  A holds r rows
     // [r, in] and B r columns [out, r]; rows and columns past r_real are zero
@@ -103,7 +109,7 @@ struct Engine {
     double wg_elems = 0;
     size_t wg_cursor = 0;
     // SwiGLU backward fused with the gate/up LoRA backward (rank 16, both
-    // pairs on, BT and I multiples of 64): its dh partials, split counts
+    // pairs on, I a multiple of 64): its dh partials, split counts
     bool silu_fused = false;
     int sl_st = 0, sl_so = 0;
     float* dh_part = nullptr;
@@ -199,11 +205,22 @@ static int alloc(Engine* e, T** p, int64_t n, const char* name, int is_f32 = -1)
     return 0;
 }
 
+// alloc of a BF16 [BT, width] buffer with BTp rows, those past BT zero; the
+// named buffer is its first BT rows.
+static int alloc_rows(Engine* e, bf16** p, int64_t width, const char* name, bool named) {
+    CK(alloc(e, p, (int64_t)e->BTp * width, name));
+    if (e->BTp > e->BT)
+        TA_HIP(hipMemsetAsync(*p + (int64_t)e->BT * width, 0,
+                              (size_t)(e->BTp - e->BT) * width * sizeof(bf16), e->s));
+    if (named) e->named[name] = {(void*)*p, {(int64_t)e->BT * width, 0}};
+    return 0;
+}
+
 // Token splits of the gB partials when go_lora makes a group's dh and gB
-// (rank 16, every on-pair's output a multiple of 64, BT a multiple of 32);
+// (rank 16, every on-pair's output a multiple of 64);
 // 0 when the group runs the per-pair kernels.  Used by the plan and the step.
 static int go_group_splits(Engine* e, const Layer& ly, std::initializer_list<int> group) {
-    if (e->r != 16 || e->BT % 32 != 0) return 0;
+    if (e->r != 16) return 0;
     int ntot = 0;
     for (int p : group) {
         if (!ly.pr[p].on) continue;
@@ -212,7 +229,7 @@ static int go_group_splits(Engine* e, const Layer& ly, std::initializer_list<int
     }
     if (!ntot) return 0;
     int s_t = 0, s_o = 0;
-    if (go_lora_splits(e->BT, ntot, &s_t, &s_o)) return 0;
+    if (go_lora_splits(e->BTp, ntot, &s_t, &s_o)) return 0;
     return s_t;
 }
 
@@ -286,7 +303,7 @@ static int engine_alloc(Engine* e) {
         for (int q = 0; q < NPAIR; q++) {
             CK(alloc(e, &ly.W[q], (int64_t)outs[q] * ins[q], "w"));
             CK(alloc(e, &ly.Wt[q], (int64_t)outs[q] * ins[q], "wt"));
-            if (ly.pr[q].on) CK(alloc(e, &ly.pr[q].h, (int64_t)BT * r, "lora.h"));
+            if (ly.pr[q].on) CK(alloc_rows(e, &ly.pr[q].h, r, "lora.h", false));
         }
         if (I % 128 == 0) CK(alloc(e, &ly.Wgu, (int64_t)2 * I * H, "wgu"));
         CK(alloc(e, &ly.res_in, (int64_t)BT * H, (p + "res_in").c_str(), 0));
@@ -313,14 +330,16 @@ static int engine_alloc(Engine* e) {
         CK(alloc(e, &ly.res_mid, (int64_t)BT * H, (p + "res_mid").c_str(), 0));
         CK(alloc(e, &ly.post_rms, BT, (p + "post_rms").c_str(), 1));
         CK(alloc(e, &ly.xn2, (int64_t)BT * H, (p + "x_normed2").c_str(), 0));
-        CK(alloc(e, &ly.gate, (int64_t)BT * I, (p + "gate").c_str(), 0));
-        CK(alloc(e, &ly.up, (int64_t)BT * I, (p + "up").c_str(), 0));
+        CK(alloc_rows(e, &ly.gate, I, (p + "gate").c_str(), true));
+        CK(alloc_rows(e, &ly.up, I, (p + "up").c_str(), true));
         CK(alloc(e, &ly.act, (int64_t)BT * I, (p + "act").c_str(), 0));
     }
-    e->silu_fused = r == 16 && BT % 64 == 0 && I % 64 == 0;
+    // (a padded batch also needs the down pair's dh rows past BT, which only
+    // go_lora writes: H a multiple of 64)
+    e->silu_fused = r == 16 && I % 64 == 0 && (e->BTp == BT || H % 64 == 0);
     if (e->silu_fused) {
-        CK(silu_lora_splits(BT, I, &e->sl_st, &e->sl_so));
-        CK(alloc(e, &e->dh_part, (int64_t)e->sl_so * 2 * BT * 16, "lora.dh_partials"));
+        CK(silu_lora_splits(e->BTp, I, &e->sl_st, &e->sl_so));
+        CK(alloc(e, &e->dh_part, (int64_t)e->sl_so * 2 * e->BTp * 16, "lora.dh_partials"));
     }
     // weight-gradient jobs in the order lora_group_bwd issues them: layers
     // L-1..0; groups down, gate/up, o, q/k/v; per group gB of each on-pair,
@@ -390,7 +409,7 @@ static int engine_alloc(Engine* e) {
     {
         // go_lora partials: [column blocks][3][BT][16] for the widest group
         const int wide = std::max(std::max(H, qd + 2 * kvd), 2 * I);
-        CK(alloc(e, &e->go_part, (int64_t)((wide + 511) / 512) * 3 * BT * 16, "lora.go_partials"));
+        CK(alloc(e, &e->go_part, (int64_t)((wide + 511) / 512) * 3 * e->BTp * 16, "lora.go_partials"));
     }
     CK(alloc(e, &e->x_final, (int64_t)BT * H, "x_final", 0));
     CK(alloc(e, &e->final_rms, BT, "final_rms", 1));
@@ -398,21 +417,22 @@ static int engine_alloc(Engine* e) {
     CK(alloc(e, &e->logits, (int64_t)BT * V, "logits", 0));
     CK(alloc(e, &e->loss_tok, BT, "loss_tok", 1));
     if (e->ce_in_dx) CK(alloc(e, &e->lse2, BT, "lse2", 1));
-    CK(alloc(e, &e->g_res, (int64_t)BT * H, "grad", 0));
+    CK(alloc_rows(e, &e->g_res, H, "grad", true));
     CK(alloc(e, &e->dres, (int64_t)BT * H, "dres", 0));
     CK(alloc(e, &e->tmpH, (int64_t)BT * H, "tmpH", 0));
-    CK(alloc(e, &e->dact, (int64_t)BT * I, "dact", 0));
-    CK(alloc(e, &e->dgate, (int64_t)BT * I, "dgate", 0));
-    CK(alloc(e, &e->dup, (int64_t)BT * I, "dup", 0));
+    CK(alloc_rows(e, &e->dact, I, "dact", true));
+    CK(alloc_rows(e, &e->dgate, I, "dgate", true));
+    CK(alloc_rows(e, &e->dup, I, "dup", true));
     CK(alloc(e, &e->dxn2, (int64_t)BT * H, "dx_normed2", 0));
     CK(alloc(e, &e->dao, (int64_t)BT * qd, "dattn_out", 0));
-    CK(alloc(e, &e->dQ, (int64_t)BT * qd, "dQ", 0));
-    CK(alloc(e, &e->dK, (int64_t)BT * kvd, "dK", 0));
-    CK(alloc(e, &e->dV, (int64_t)BT * kvd, "dV", 0));
+    CK(alloc_rows(e, &e->dQ, qd, "dQ", true));
+    CK(alloc_rows(e, &e->dK, kvd, "dK", true));
+    CK(alloc_rows(e, &e->dV, kvd, "dV", true));
     CK(alloc(e, &e->dxn, (int64_t)BT * H, "dx_normed", 0));
     CK(alloc(e, &e->delta, (int64_t)BT * maxout, "delta", 0));
     CK(alloc(e, &e->dh, (int64_t)BT * r, "dh", 0));
-    CK(alloc(e, &e->dh_cat, (int64_t)BT * r * 3, "dh_cat", 0));
+    CK(alloc(e, &e->dh_cat, (int64_t)e->BTp * r * 3, "dh_cat"));
+    e->named["dh_cat"] = {(void*)e->dh_cat, {(int64_t)BT * r * 3, 0}};
     CK(alloc(e, &e->Dbuf, attn_bwd_rowbuf_floats(e->B, e->T, c.n_q), "Dbuf", 1));
     CK(alloc(e, &e->dkv_part, (int64_t)2 * e->B * c.n_q * e->T * c.head_dim, "dkv_part", 1));
     e->rope_bwd = rope_table(e->T, c.head_dim, c.rope_theta, -1.f, e->s);
@@ -568,7 +588,7 @@ static int lora_group_bwd(Engine* e, Layer& ly, std::initializer_list<int> group
             fl += 2.0 * gflops(dBT, r, pr.out);
         }
         TIMED(TA_CAT_LORA, fl, bytes,
-              go_lora(go_on, ld, bt, hs, parts, outs, n, BT, e->go_part, e->dh_cat, ldh, e->s));
+              go_lora(go_on, ld, bt, hs, parts, outs, n, e->BTp, e->go_part, e->dh_cat, ldh, e->s));
     }
     for (int q = 0; q < n && !dh_ready && go_group_splits(e, ly, group) == 0; q++) {
         Pair& pr = ly.pr[on[q]];
@@ -808,9 +828,9 @@ static int backward(Engine* e) {
                   dBT * I * 10 + dBT * 96,
                   silu_bwd_lora(e->dact, ly.gate, ly.up, e->dgate, e->dup, e->shadowT + PRg.offB,
                                 e->shadowT + PRu.offB, PRg.h, PRu.h, e->dh_part, pg, pu,
-                                ga_down ? e->dh_cat : nullptr, ga_down, BT, I, s));
+                                ga_down ? e->dh_cat : nullptr, ga_down, e->BTp, I, s));
             TIMED(TA_CAT_LORA, 0, dBT * 128.0 * e->sl_so + dBT * 64,
-                  dh_reduce2(e->dh_part, e->sl_so, BT, e->dh_cat, 2 * e->r, s));
+                  dh_reduce2(e->dh_part, e->sl_so, e->BTp, e->dh_cat, 2 * e->r, s));
         } else {
             TIMED(TA_CAT_ELEMWISE, 0, dBT * I * 10,
                   ta_silu_mul_bwd(e->dact, ly.gate, ly.up, e->dgate, e->dup, (int64_t)BT * I, s));
@@ -1051,6 +1071,7 @@ void* ta_engine_create_ex(const ta_model_config* mc, const ta_adapt_config* ac, 
     e->B = B;
     e->T = T;
     e->BT = B * T;
+    e->BTp = (e->BT + 63) / 64 * 64;
     e->H = mc->hidden;
     e->qd = mc->n_q * mc->head_dim;
     e->kvd = mc->n_kv * mc->head_dim;
