@@ -149,8 +149,11 @@ __global__ __launch_bounds__(1024) void k_cross_entropy_reg(const bf16* __restri
     // a target outside [0, V) reads nothing (the reference would read out of
     // bounds for tgt >= V; ids come from a vocab-sized tokenizer)
     const bool hit = tgt >= 0 && tgt < V;
-    // (read before the block's first barrier: dlogits may overwrite the row)
-    const float tl = hit ? bf2f(((const bf16*)L)[tgt]) : 0.f;
+    // read before the block's first barrier: dlogits may overwrite the row (the
+    // empty asm statement pins the value here, where the compiler, told that
+    // logits and dlogits are restrict, could otherwise sink the load)
+    float tl = hit ? bf2f(((const bf16*)L)[tgt]) : 0.f;
+    asm volatile("" : "+v"(tl));
     bf16x8v r[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
