@@ -2084,9 +2084,86 @@ static double segment_us(int M, int N, int ksteps, bool lora) {
     return std::min(deep, split256_us(M, N, ksteps, t, sp, lora));
 }
 
+// Splits of a long K over few 256-row tiles: as many as keep the blocks within
+// one per CU, at least 8 stages each.
+static int split256_for(int tiles, int ksteps) {
+    return std::max(1, std::min(256 / tiles, ksteps / 8));
+}
+// The 256-row kernels' width for such a split: the one with the most blocks
+// (256-wide on a tie).
+static int split256_variant(int M, int N, int ksteps) {
+    const int t192 = ceil_div(M, 256) * ceil_div(N, 192);
+    const int t256 = ceil_div(M, 256) * ceil_div(N, 256);
+    return t192 * split256_for(t192, ksteps) > t256 * split256_for(t256, ksteps) ? 17 : 18;
+}
+static bool is_big_shape(int M, int N, int ksteps) {
+    return (M >= 1024 && N >= 1024) || (M >= 256 && N >= 128 && ksteps >= 32);
+}
+
+// The 128-row form of a K-contiguous product, if one takes it: k_gemm_deep
+// (deep.bn != 0) when one 128-row tile per CU covers the output (and a long K
+// does not run faster in the 256-row kernels' splits), else k_gemm_mid (mid
+// != 0).  may_split false: the product must run in one pass over K.
+struct SmallPlan {
+    DeepPlan deep;
+    int mid = 0;
+};
+static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split, bool capturing) {
+    SmallPlan p;
+    p.mid = mid_bn(M, N, N > 3072 ? 256 : 192, ksteps, M >= 1024 && N >= 1024, 128);
+    const bool big = p.mid == 0 && is_big_shape(M, N, ksteps);
+    // (a capture of a shape that no other form splits takes no pointer
+    // into the scratch pool, which may move before a replay)
+    const bool fresh_split = M >= 128 && !big;
+    p.deep = deep_plan(M, N, ksteps, may_split, 128);
+    if (p.deep.bn && p.deep.splits > 1 && fresh_split && capturing)
+        p.deep = deep_plan(M, N, ksteps, false, 128);
+    if (p.deep.bn && big) {
+        const int bn = big_bn(split256_variant(M, N, ksteps));
+        const int t = ceil_div(M, 256) * ceil_div(N, bn);
+        if (p.deep.us > 0.97 * split256_us(M, N, ksteps, t, split256_for(t, ksteps), lora))
+            p.deep.bn = 0;
+    }
+    return p;
+}
+
+// Kernel variant of the 256-row tiles.
+static int big_variant(int M, int N, int ksteps, bool may_split) {
+    if (may_split && ksteps >= 32 && ceil_div(M, 256) * ceil_div(N, N > 3072 ? 256 : 192) < 192)
+        return split256_variant(M, N, ksteps);
+    if (N > 3072) return 18;
+    // up to N = 3072 the 256-wide tiles when they need fewer waves of 256
+    // blocks (waves x tile area): N = 2048 at M = 8192 is one wave of
+    // 256-wide tiles against 1.4 of 192-wide (48 against 73 us measured)
+    const int64_t tm = ceil_div(M, 256);
+    const int64_t w192 = (tm * ceil_div(N, 192) + 255) / 256;
+    const int64_t w256 = (tm * ceil_div(N, 256) + 255) / 256;
+    return w256 * 256 < w192 * 192 ? 18 : 17;
+}
+
+// Columns before the tail of a product on 256 x 256 tiles (0: no tail).  A
+// last wave of at most half the CUs' blocks (M 8192 x N 8960: 4.375 waves)
+// runs as its own launch of 128-row tiles, two blocks per CU at a quarter of
+// the work each: the columns past the last whole wave go to k_gemm_deep or
+// k_gemm_mid.  That launch runs unsplit (small_plan with may_split false), so
+// every output element keeps its k order and the result is the same, and the
+// LoRA terms, which exist for it only in the epilogues' layout, are fused.
+static int tail_main_cols(int M, int N, int ksteps) {
+    const int tiles_m = ceil_div(M, 256), tiles = tiles_m * ceil_div(N, 256);
+    const int full = tiles / 256, rem = tiles % 256;
+    if (full < 1 || rem == 0 || rem > 128 || (full * 256) % tiles_m != 0) return 0;
+    const int n_main = full * 256 / tiles_m * 256;
+    return n_main > 3072 && n_main < N && mid_bn(M, N - n_main, 256, ksteps, false, 128) != 0
+               ? n_main
+               : 0;
+}
+
 // Shape-driven dispatch.  lora (may be NULL): rank-r terms applied to C after the base epilogue, fused
 // into the large-GEMM kernel's epilogue when that kernel runs unsplit and
-// applied by k_rank_update right after the GEMM otherwise.
+// applied by k_rank_update right after the GEMM otherwise.  force_splits: 0
+// picks the splits of K, kUnsplit picks among the forms that take K in one
+// pass, above 0 that many splits.
+constexpr int kUnsplit = -1;
 int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16* X, int64_t ldx,
                   const bf16* Y, int64_t ldy, float beta, void* C, int64_t ldc, const bf16* bias,
                   hipStream_t s, int force_splits, const LoraEpi* lora) {
@@ -2143,16 +2220,8 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         }
     };
     const int ksteps = (K + BK - 1) / BK;
-    const int t192 = ((M + 255) / 256) * ((N + 191) / 192);
-    const int t256 = ((M + 255) / 256) * ((N + 255) / 256);
-    // split-K over few 256-row tiles: as many splits as keep the blocks within
-    // one per CU (at least 8 stages each), with the tile width that gives the
-    // most blocks (256-wide on a tie)
-    auto split_for = [&](int tiles) { return std::max(1, std::min(256 / tiles, ksteps / 8)); };
-    const int split_variant = t192 * split_for(t192) > t256 * split_for(t256) ? 17 : 18;
     const bool auto_form = g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0;
-    const bool big_shape =
-        (M >= 1024 && N >= 1024) || (M >= 256 && N >= 128 && ksteps >= 32);
+    const bool big_shape = is_big_shape(M, N, ksteps);
     // K a LoRA rank (at most 64): k_gemm_rank.  The 128-row tiles below would
     // stage 64 k of zeros and write C two bytes at a time (8192 x 1536 x 16:
     // 22 us, and 48 us with beta 1 and a K-strided Y)
@@ -2195,28 +2264,16 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         }
         return check_launch("gemm");
     }
-    // K-contiguous BF16 GEMMs too small to fill the chip with 256-row tiles:
-    // k_gemm_deep when one 128-row tile per CU covers the output (and a long K
-    // does not run faster in the 256-row kernels' splits), else k_gemm_mid
-    // (LoRA terms in the epilogue of both)
+    // K-contiguous BF16 GEMMs too small to fill the chip with 256-row tiles
+    // (LoRA terms in the epilogue of both forms)
     if (pipe_ok && (auto_form || g_big_variant == 19 || g_big_variant == 20)) {
-        const int bn = g_big_variant == 19   ? 128
-                       : g_big_variant == 20 ? 64
-                                             : mid_bn(M, N, N > 3072 ? 256 : 192, ksteps,
-                                                      M >= 1024 && N >= 1024, 128);
-        DeepPlan dp;
-        if (auto_form) {
-            // (a capture of a shape that no other form splits takes no pointer
-            // into the scratch pool, which may move before a replay)
-            const bool fresh_split = M >= 128 && !(bn == 0 && big_shape);
-            dp = deep_plan(M, N, ksteps, true, 128);
-            if (dp.bn && dp.splits > 1 && fresh_split && is_capturing(s))
-                dp = deep_plan(M, N, ksteps, false, 128);
-            if (dp.bn && bn == 0 && big_shape) {
-                const int t = split_variant == 17 ? t192 : t256;
-                if (dp.us > 0.97 * split256_us(M, N, ksteps, t, split_for(t), lora_on)) dp.bn = 0;
-            }
-        }
+        SmallPlan sp;
+        if (auto_form)
+            sp = small_plan(M, N, ksteps, lora_on, force_splits != kUnsplit, is_capturing(s));
+        else
+            sp.mid = g_big_variant == 19 ? 128 : 64;
+        const DeepPlan& dp = sp.deep;
+        const int bn = sp.mid;
         if (dp.bn) {
             a.tiles_m = (M + 127) / 128;
             a.tiles_n = (N + dp.bn - 1) / dp.bn;
@@ -2278,19 +2335,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     // split-K when K is long: 32 or more 64-k stages)
     if (pipe_ok && (big_shape || (g_big_variant != 0 && M >= 256 && N >= 128))) {
         int variant = g_big_variant;
-        if (variant == 0) variant = N > 3072 ? 18 : 17;
-        // up to N = 3072 the 256-wide tiles when they need fewer waves of 256
-        // blocks (waves x tile area): N = 2048 at M = 8192 is one wave of
-        // 256-wide tiles against 1.4 of 192-wide (48 against 73 us measured)
-        if (g_big_variant == 0 && N <= 3072) {
-            const int64_t tm = (M + 255) / 256;
-            const int64_t w192 = (tm * ((N + 191) / 192) + 255) / 256;
-            const int64_t w256 = (tm * ((N + 255) / 256) + 255) / 256;
-            if (w256 * 256 < w192 * 192) variant = 18;
-        }
-        const bool auto_split = force_splits <= 0 && g_force_splits == 0 && ksteps >= 32;
-        if (g_big_variant == 0 && auto_split && (N > 3072 ? t256 : t192) < 192)
-            variant = split_variant;
+        if (variant == 0) variant = big_variant(M, N, ksteps, auto_form);
         const int BNb = big_bn(variant);
         a.tiles_m = (M + 255) / 256;
         a.tiles_n = (N + BNb - 1) / BNb;
@@ -2300,39 +2345,27 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
             splits = force_splits;
         else if (g_force_splits > 0)
             splits = g_force_splits;
-        else if (tiles < 192 && ksteps >= 32)
-            splits = split_for(tiles);
+        else if (tiles < 192 && ksteps >= 32 && force_splits != kUnsplit)
+            splits = split256_for(tiles, ksteps);
         if (splits < 1) splits = 1;
-        // A last wave of at most half the CUs' blocks (M 8192 x N 8960: 4.375
-        // waves of 256 x 256 tiles) runs as its own launch of 128-row tiles,
-        // two blocks per CU at a quarter of the work each: the columns past
-        // the last whole wave of 256-wide tiles go to k_gemm_mid.  Every
-        // output element keeps its k order, so the result is the same.
-        if (g_big_variant == 0 && force_splits <= 0 && g_force_splits == 0 && splits == 1 &&
-            variant == 18) {
-            const int full = tiles / 256, rem = tiles % 256;
-            if (full >= 1 && rem > 0 && rem <= 128 && (full * 256) % a.tiles_m == 0) {
-                const int n_main = full * 256 / a.tiles_m * 256;
-                if (n_main > 3072 && n_main < N &&
-                    mid_bn(M, N - n_main, 256, ksteps, false, 128) != 0) {
-                    const bool fz = lora && lora->n > 0;
-                    LoraEpi lt{};
-                    if (fz) {
-                        lt = *lora;
-                        for (int p = 0; p < lora->n; p++) {
-                            lt.v_nk[p] = lora->v_nk[p] + (int64_t)n_main * lora->r;
-                            lt.v_alt[p] = nullptr;  // the mid kernel fuses every rank here
-                        }
-                    }
-                    int rc = gemm_dispatch(xk, yk, M, n_main, K, alpha, X, ldx, Y, ldy, beta, C,
-                                           ldc, bias, s, 0, lora);
-                    if (rc) return rc;
-                    return gemm_dispatch(xk, yk, M, N - n_main, K, alpha, X, ldx,
-                                         Y + (int64_t)n_main * ldy, ldy, beta,
-                                         (bf16*)C + n_main, ldc, bias ? bias + n_main : nullptr,
-                                         s, 0, fz ? &lt : nullptr);
+        const int n_main =
+            auto_form && splits == 1 && variant == 18 ? tail_main_cols(M, N, ksteps) : 0;
+        if (n_main) {
+            LoraEpi lt{};
+            if (lora_on) {
+                lt = *lora;
+                for (int p = 0; p < lora->n; p++) {
+                    lt.v_nk[p] = lora->v_nk[p] + (int64_t)n_main * lora->r;
+                    lt.v_alt[p] = nullptr;  // (its rows are N apart: no tail of it)
                 }
             }
+            int rc = gemm_dispatch(xk, yk, M, n_main, K, alpha, X, ldx, Y, ldy, beta, C, ldc, bias,
+                                   s, 0, lora);
+            if (rc) return rc;
+            return gemm_dispatch(xk, yk, M, N - n_main, K, alpha, X, ldx,
+                                 Y + (int64_t)n_main * ldy, ldy, beta, (bf16*)C + n_main, ldc,
+                                 bias ? bias + n_main : nullptr, s, kUnsplit,
+                                 lora_on ? &lt : nullptr);
         }
         int steps_per = (ksteps + splits - 1) / splits;
         a.k_per_split = steps_per * BK;
@@ -2420,7 +2453,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     int splits = 1;
     if (force_splits > 0) {
         splits = force_splits;
-    } else if (tiles < 256 && ksteps >= 16) {
+    } else if (tiles < 256 && ksteps >= 16 && force_splits != kUnsplit) {
         splits = (512 + tiles - 1) / tiles;
         if (splits > ksteps / 4) splits = ksteps / 4;
         if (splits < 1) splits = 1;
@@ -2910,6 +2943,34 @@ int ta_gemm_rm(int x_kmajor, int y_kmajor, int M, int N, int K, float alpha, con
                "gemm_rm: M/N/K and leading dims must be > 0");
     return gemm_dispatch(x_kmajor != 0, y_kmajor != 0, M, N, K, alpha, X, ldx, Y, ldy, beta, C,
                          ldc, bias, (hipStream_t)stream, 0, nullptr);
+}
+
+int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
+    TA_REQUIRE(M > 0 && N > 0 && K > 0 && K % BK == 0 && out,
+               "gemm_plan: M, N, K > 0 and K a multiple of %d", BK);
+    const int ks = K / BK;
+    for (int i = 0; i < 8; i++) out[i] = 0;
+    auto small = [&](int n, const SmallPlan& p, int32_t* o) {
+        o[0] = n;
+        o[1] = p.deep.bn ? TA_GEMM_DEEP : p.mid ? TA_GEMM_MID : TA_GEMM_TILES;
+        o[2] = p.deep.bn ? p.deep.bn : p.mid;
+        o[3] = p.deep.bn ? p.deep.splits : 1;
+        return o[1] != TA_GEMM_TILES;
+    };
+    if (small(N, small_plan(M, N, ks, lora != 0, true, captured != 0), out) ||
+        !is_big_shape(M, N, ks))
+        return 0;
+    const int variant = big_variant(M, N, ks, true), bn = big_bn(variant);
+    const int tiles = ceil_div(M, 256) * ceil_div(N, bn);
+    out[1] = TA_GEMM_BIG;
+    out[2] = bn;
+    out[3] = tiles < 192 && ks >= 32 ? split256_for(tiles, ks) : 1;
+    const int n_main = out[3] == 1 && variant == 18 ? tail_main_cols(M, N, ks) : 0;
+    if (n_main) {
+        out[0] = n_main;
+        small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, false, captured != 0), out + 4);
+    }
+    return 0;
 }
 
 int ta_gemm_rm_variant(int variant, int x_kmajor, int y_kmajor, int M, int N, int K, float alpha,

@@ -991,6 +991,7 @@ int lora_rank_update(bool delta, bf16* Y, int64_t ldy, int M, int N, int r, floa
         p.u[i] = U[i];
         p.ldu[i] = ldu[i];
         p.y[i] = V[i];
+        TA_REQUIRE(U[i] && V[i], "lora_rank_update: null operand");
         TA_REQUIRE(((uintptr_t)U[i] & 15) == 0 && (ldu[i] & 7) == 0,
                    "lora_rank_update: U rows must be 16-byte aligned");
     }

@@ -1,0 +1,57 @@
+"""The choice of kernel forms for K-contiguous GEMMs (ta_gemm_plan: host
+arithmetic, no GPU).
+
+A product on 256 x 256 tiles whose last wave is nearly empty runs its last
+columns as a second launch.  The LoRA terms of that launch exist only in the
+layout the fused epilogues read, so it must not split K: a split leaves them
+to a pass of its own, which needs the other layout.
+"""
+import ctypes
+
+import pytest
+
+import tadapt
+
+TILES, DEEP, MID, BIG = range(4)
+
+
+def plan(M, N, K, lora=1, captured=0):
+    out = (ctypes.c_int32 * 8)()
+    tadapt.call("ta_gemm_plan", M, N, K, lora, captured, ctypes.addressof(out))
+    rows = [tuple(out[:4]), tuple(out[4:])]
+    return [r for r in rows if r[0]]
+
+
+def widths(M):
+    """Output widths around every last wave of 256-wide tiles of at most half
+    the CUs, up to 20,480 columns."""
+    tm = (M + 255) // 256
+    for full in range(1, 20480 // 256 * tm // 256 + 1):
+        if full * 256 % tm:
+            continue
+        main = full * 256 // tm * 256
+        for over in (64, 72, 120, 128, 136, 256, 448, 1000, 2048, 4096):
+            if main + over <= 20480:
+                yield main + over
+
+
+@pytest.mark.parametrize("M", [256, 777, 1024, 2048, 2331, 4096, 6144, 8192, 16384])
+def test_tail_never_splits(M):
+    tails = 0
+    for N in widths(M):
+        for K in [64 * k for k in (2, 7, 14, 18, 24, 31, 32, 40, 56, 76, 140, 296)]:
+            rows = plan(M, N, K)
+            assert sum(r[0] for r in rows) == N, (M, N, K, rows)
+            if len(rows) == 2:
+                tails += 1
+                assert rows[0][1] == BIG and rows[0][3] == 1, (M, N, K, rows)
+                # and one of the forms whose epilogue takes the LoRA terms
+                assert rows[1][1] in (DEEP, MID) and rows[1][3] == 1, (M, N, K, rows)
+    assert tails or M in (256, 777, 2331)
+
+
+def test_tail_of_a_wide_intermediate():
+    """2048 tokens, hidden 1536, intermediate 8320, down_proj adapted: 264
+    tiles, of which the last 128 columns run apart."""
+    rows = plan(2048, 8320, 1536)
+    assert len(rows) == 2 and rows[1] == (128, DEEP, 64, 1), rows
