@@ -22,6 +22,7 @@
 
 #include <mutex>
 
+#include "kmeans_stop.hpp"
 #include "ta_internal.hpp"
 
 // Partial rows of ta_centroid_accumulate_bf16_noalloc, in a file-scope device
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(64) void k_kmeans_rows(const float* __restrict__ X,
     if (n < N) out[(int64_t)r * N + n] = d;
     if (k > 0 && blockIdx.y == 0) {
         for (int i = threadIdx.x; i < D; i += 64) C[(int64_t)r * D + i] = X[(int64_t)row * D + i];
-        if (r == 0 && threadIdx.x == 0) *done = 0;
+        if (r == 0 && threadIdx.x == 0) *done = kKmeansRunning;
     }
 }
 
@@ -619,7 +620,7 @@ __global__ __launch_bounds__(1024) void k_kmeans_seed(const float* __restrict__ 
         if (first >= N) first = N - 1;
         if (lane == 0) {
             chosen[0] = last = first;
-            *done = 0;
+            *done = kKmeansRunning;
         }
     }
     for (int n = threadIdx.x; n < N; n += 1024) d2[n] = FLT_MAX;
@@ -738,8 +739,7 @@ __device__ __forceinline__ int nearest64(const float* __restrict__ dist, int N, 
 // and the new center's distances into dout.  An empty center becomes zero
 // (REF, the reference's loop) or stays.  A pass that changes no assignment
 // ends the loop: the centers and distances of every later pass would be the
-// same values, so *done makes later launches return at once.  (A block of
-// the same launch that sees it early skips what is unchanged anyway.)
+// same values, so *done makes later launches return at once.
 // asg_in / asg_out: the previous and this pass's assignments (REF's first
 // pass compares against zeros); asg_fin always holds the latest.
 template <bool REF>
@@ -753,7 +753,10 @@ __global__ __launch_bounds__(256) void k_kmeans_iter(
     __shared__ int si[4][64];
     __shared__ __attribute__((aligned(16))) float cen[kIterC];
     __shared__ uint64_t smask[64];
-    if (*(volatile int32_t*)done) return;
+    // (block 0 may store while others read: either value gives this launch the
+    // same answer)
+    if (kmeans_stopped(__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), it))
+        return;
     const int c = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nb = (N + 63) / 64;
     // members of c, a bit per snapshot (in LDS up to 4096 snapshots)
@@ -776,7 +779,8 @@ __global__ __launch_bounds__(256) void k_kmeans_iter(
     if (!changed) {
         if (c == 0 && threadIdx.x == 0) {
             if (REF && iters_out) *iters_out = it;
-            *done = 1;
+            __hip_atomic_store(done, kmeans_stop_after(it), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -824,7 +828,7 @@ __global__ __launch_bounds__(64) void k_kmeans_cdist(const float* __restrict__ X
                                                      const float* __restrict__ C, int N, int D,
                                                      float* __restrict__ dist,
                                                      const int32_t* __restrict__ done) {
-    if (*done) return;
+    if (*done != kKmeansRunning) return;
     const int c = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
     const float d = sqdist_col(XT, N, D, min(n, N - 1), C + (int64_t)c * D);
     if (n < N) dist[(int64_t)c * N + n] = d;
@@ -851,7 +855,7 @@ __global__ __launch_bounds__(1024) void k_kmeans_rank(const float* __restrict__ 
     __shared__ float sw[1024];
     __shared__ int sa[1024];
     const int t = threadIdx.x;
-    const bool have = *done != 0;
+    const bool have = *done != kKmeansRunning;
     double m = 0.0;
     for (int n0 = 0; n0 < N; n0 += 1024) {
         const int n = n0 + t, cnt = min(1024, N - n0);
