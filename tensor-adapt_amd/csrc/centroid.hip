@@ -20,6 +20,7 @@
 // iters, so the launches always drain.
 #include <float.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "kmeans_stop.hpp"
@@ -501,16 +502,22 @@ __global__ __launch_bounds__(1024) void k_kmeans_ref(const float* __restrict__ X
 // distances of longer centers
 constexpr int kIterC = 4096;
 
-// XT[d][n] = X[n][d], 32 x 32 tiles
+// XT[d][n] = X[n][d], 32 x 32 tiles in one grid dimension (N or D alone may
+// need more tiles than the other dimensions take)
 __global__ __launch_bounds__(256) void k_kmeans_transpose(const float* __restrict__ X,
                                                           float* __restrict__ XT, int N, int D) {
     __shared__ float t[32][33];
-    const int n0 = blockIdx.x * 32, d0 = blockIdx.y * 32, c = threadIdx.x & 31;
-    for (int r = threadIdx.x >> 5; r < 32; r += 8)
-        if (n0 + r < N && d0 + c < D) t[r][c] = X[(int64_t)(n0 + r) * D + d0 + c];
-    __syncthreads();
-    for (int r = threadIdx.x >> 5; r < 32; r += 8)
-        if (d0 + r < D && n0 + c < N) XT[(int64_t)(d0 + r) * N + n0 + c] = t[c][r];
+    const int64_t td = (D + 31) / 32, tiles = td * ((N + 31) / 32);
+    const int c = threadIdx.x & 31;
+    for (int64_t q = blockIdx.x; q < tiles; q += gridDim.x) {
+        const int n0 = (int)(q / td) * 32, d0 = (int)(q % td) * 32;
+        for (int r = threadIdx.x >> 5; r < 32; r += 8)
+            if (n0 + r < N && d0 + c < D) t[r][c] = X[(int64_t)(n0 + r) * D + d0 + c];
+        __syncthreads();
+        for (int r = threadIdx.x >> 5; r < 32; r += 8)
+            if (d0 + r < D && n0 + c < N) XT[(int64_t)(d0 + r) * N + n0 + c] = t[c][r];
+        __syncthreads();
+    }
 }
 
 // The chain of snapshot n (column n of XT) against the D values at b (read
@@ -559,7 +566,7 @@ __device__ __forceinline__ float sqdist_col(const float* __restrict__ XT, int N,
     return d;
 }
 
-// out[r][n]: distance of snapshot n to snapshot r (block x = r, 64 snapshots
+// out[r][n]: distance of snapshot n to snapshot r (block y = r, 64 snapshots
 // per block), or, with k > 0, to the r-th of the reference's k initial
 // centers, snapshot (r N) / k, which is also copied to C[r]
 __global__ __launch_bounds__(64) void k_kmeans_rows(const float* __restrict__ X,
@@ -568,7 +575,7 @@ __global__ __launch_bounds__(64) void k_kmeans_rows(const float* __restrict__ X,
                                                     float* __restrict__ out,
                                                     int32_t* __restrict__ done) {
     __shared__ __attribute__((aligned(16))) float b[kIterC];
-    const int r = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
+    const int r = blockIdx.y, n = blockIdx.x * 64 + threadIdx.x;
     const int row = k > 0 ? (int)(((int64_t)r * N) / k) : r;
     if (D <= kIterC) {
         for (int i = threadIdx.x; i < D; i += 64) b[i] = X[(int64_t)row * D + i];
@@ -577,7 +584,7 @@ __global__ __launch_bounds__(64) void k_kmeans_rows(const float* __restrict__ X,
     const float d = D <= kIterC ? sqdist_col(XT, N, D, min(n, N - 1), b)
                                 : sqdist_col(XT, N, D, min(n, N - 1), X + (int64_t)row * D);
     if (n < N) out[(int64_t)r * N + n] = d;
-    if (k > 0 && blockIdx.y == 0) {
+    if (k > 0 && blockIdx.x == 0) {
         for (int i = threadIdx.x; i < D; i += 64) C[(int64_t)r * D + i] = X[(int64_t)row * D + i];
         if (r == 0 && threadIdx.x == 0) *done = kKmeansRunning;
     }
@@ -829,7 +836,7 @@ __global__ __launch_bounds__(64) void k_kmeans_cdist(const float* __restrict__ X
                                                      float* __restrict__ dist,
                                                      const int32_t* __restrict__ done) {
     if (*done != kKmeansRunning) return;
-    const int c = blockIdx.x, n = blockIdx.y * 64 + threadIdx.x;
+    const int c = blockIdx.y, n = blockIdx.x * 64 + threadIdx.x;
     const float d = sqdist_col(XT, N, D, min(n, N - 1), C + (int64_t)c * D);
     if (n < N) dist[(int64_t)c * N + n] = d;
 }
@@ -1027,6 +1034,9 @@ struct KmeansScratch {
         return true;
     }
 };
+static dim3 transpose_grid(int N, int D) {
+    return dim3((unsigned)std::min<int64_t>((int64_t)((N + 31) / 32) * ((D + 31) / 32), 1 << 20));
+}
 // Most passes the reference's loop launches one by one (its own cap is 50): a
 // launch after the last change still costs about 2 us, and beyond this the
 // loop on one workgroup, which stops by itself, is kept.
@@ -1097,19 +1107,19 @@ int ta_kmeans_ref(const float* snaps, int N, int D, int k, int max_iters, float*
     // from global memory below 2^17 (32 x 1536, k = 2: 127 against 130; 96 x
     // 512, k = 8: 373 against 99)
     const bool small = (int64_t)k * N * D < (int64_t(1) << ((int64_t)N * D <= kXs ? 20 : 17));
-    if (!small && max_iters > 0 && max_iters <= kRefLaunches) {
+    if (!small && max_iters > 0 && max_iters <= kRefLaunches && k <= 65535) {
         KmeansScratch m;
         TA_REQUIRE(m.get(N, D, k, 0, s), "kmeans_ref: scratch allocation failed");
-        tlaunch(k_kmeans_transpose, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), s, snaps, m.xt, N,
+        tlaunch(k_kmeans_transpose, transpose_grid(N, D), dim3(256), s, snaps, m.xt, N,
                 D);
-        tlaunch(k_kmeans_rows, dim3(k, (N + 63) / 64), dim3(64), s, snaps, m.xt, N, D, k, centers,
+        tlaunch(k_kmeans_rows, dim3((N + 63) / 64, k), dim3(64), s, snaps, m.xt, N, D, k, centers,
                 m.dist[0], m.done);
         for (int it = 0; it < max_iters; it++) {
             tlaunch(k_kmeans_iter<true>, dim3(k), dim3(256), s, snaps, m.xt, centers, N, D, k, it,
                     m.dist[it & 1], m.dist[(it + 1) & 1], m.asg[it & 1], m.asg[(it + 1) & 1],
                     assign, m.masks, m.done, iters_out, it + 1 == max_iters);
             if (D > kIterC && it + 1 < max_iters)
-                tlaunch(k_kmeans_cdist, dim3(k, (N + 63) / 64), dim3(64), s, m.xt, centers, N, D,
+                tlaunch(k_kmeans_cdist, dim3((N + 63) / 64, k), dim3(64), s, m.xt, centers, N, D,
                         m.dist[(it + 1) & 1], m.done);
         }
         return check_launch("kmeans_ref");
@@ -1140,9 +1150,9 @@ int ta_kmeans_pp(const float* snaps, const float* weights, int N, int D, int k, 
     KmeansScratch m;
     const bool pairs = N <= kPairMax;
     TA_REQUIRE(m.get(N, D, k, pairs ? N : 1, s), "kmeans_pp: scratch allocation failed");
-    tlaunch(k_kmeans_transpose, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), s, snaps, m.xt, N, D);
+    tlaunch(k_kmeans_transpose, transpose_grid(N, D), dim3(256), s, snaps, m.xt, N, D);
     if (pairs)
-        tlaunch(k_kmeans_rows, dim3(N, (N + 63) / 64), dim3(64), s, snaps, m.xt, N, D, 0, nullptr,
+        tlaunch(k_kmeans_rows, dim3((N + 63) / 64, N), dim3(64), s, snaps, m.xt, N, D, 0, nullptr,
                 m.pd, nullptr);
     tlaunch(k_kmeans_seed, dim3(1), dim3(1024), s, snaps, m.xt, pairs ? m.pd : nullptr, N, D, k,
             seed, m.d2, m.pre, m.c, m.dist[0], m.chosen, m.done);
@@ -1151,7 +1161,7 @@ int ta_kmeans_pp(const float* snaps, const float* weights, int N, int D, int k, 
                 m.dist[it & 1], m.dist[(it + 1) & 1], m.asg[it & 1], m.asg[(it + 1) & 1], m.asg[2],
                 m.masks, m.done, nullptr, false);
         if (D > kIterC)
-            tlaunch(k_kmeans_cdist, dim3(k, (N + 63) / 64), dim3(64), s, m.xt, m.c, N, D,
+            tlaunch(k_kmeans_cdist, dim3((N + 63) / 64, k), dim3(64), s, m.xt, m.c, N, D,
                     m.dist[(it + 1) & 1], m.done);
     }
     tlaunch(k_kmeans_rank, dim3(1), dim3(1024), s, weights, N, D, k, m.dist[iters & 1], m.c,

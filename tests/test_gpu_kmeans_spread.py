@@ -96,3 +96,24 @@ def test_few_passes_match_the_loop():
         for c, a, i in got:
             assert np.array_equal(c.reshape(8, 64), want_c)
             assert np.array_equal(a, asg) and int(i[0]) == n_it
+
+
+@pytest.mark.parametrize("pp", [True, False])
+@pytest.mark.parametrize("N,D,k", [(2, 2_200_000, 2), (64 * 65536 + 10, 1, 2)])
+def test_more_blocks_than_a_small_grid_dimension(N, D, k, pp):
+    """Dimensions and snapshot counts beyond 65,535 tiles or blocks: the grids
+    put them in x."""
+    X, W = data(N, D, "dups")
+    C = torch.empty(k * D, device=DEV)
+    A = torch.empty(N, dtype=torch.int32, device=DEV)
+    it = torch.empty(1, dtype=torch.int32, device=DEV)
+    if pp:
+        call("ta_kmeans_pp", P(dev(X)), P(dev(W)), N, D, k, 2, ctypes.c_uint64(5), P(C), P(A),
+             None, None, S())
+        rc, ra = O.kmeans_pp(X, W, k, 2, 5)[:2]
+    else:
+        call("ta_kmeans_ref", P(dev(X)), N, D, k, 50, P(C), P(A), P(it), S())
+        rc, ra, ri = O.kmeans_ref(X, k)
+        assert int(host(it)[0]) == ri
+    assert np.array_equal(host(A), ra)
+    assert np.array_equal(host(C).reshape(k, D), rc)
