@@ -1037,10 +1037,31 @@ struct KmeansScratch {
 static dim3 transpose_grid(int N, int D) {
     return dim3((unsigned)std::min<int64_t>((int64_t)((N + 31) / 32) * ((D + 31) / 32), 1 << 20));
 }
-// Most passes the reference's loop launches one by one (its own cap is 50): a
-// launch after the last change still costs about 2 us, and beyond this the
-// loop on one workgroup, which stops by itself, is kept.
-constexpr int kRefLaunches = 128;
+// Whether the reference's loop runs as one launch per pass.  Nothing tells the
+// host that the data has settled, so every pass up to the cap is launched, at
+// 3.7 us each when it has nothing left to do (twice that with
+// k_kmeans_cdist); the loop on one workgroup stops by itself, at pass_us a
+// pass (within a factor of 1.7 of 27 of 28 measured sizes).
+// Launches where three passes of the loop cost as much: data that settles in
+// the second pass, the first that can end it, then loses a little, and data
+// that settles later gains.  64 x 512, k = 32: cap 25 87 or 168 us in the loop
+// (settling in two passes or in five), 101 or 107 launched; cap 50, where the
+// loop stays, 200 launched.  96 x 1536, k = 4, cap 50: 376 or 1160 against 195
+// or 336.  Caps below 25 count as 25 and small work stays in the loop: k N D
+// below 2^20 with the snapshots in its LDS (64 x 512, k = 16, cap 25: 78 or 150
+// against 103 or 96), below 2^17 without (32 x 1536, k = 2: 127 or 193 against
+// 107 or 139).
+static bool ref_launched(int N, int D, int k, int max_iters) {
+    const bool lds = (int64_t)N * D <= kXs;
+    if (max_iters <= 0 || max_iters > 128 || k > 65535 ||
+        (int64_t)k * N * D < (int64_t(1) << (lds ? 20 : 17)))
+        return false;
+    const double units = (double)k * (((int64_t)N + 63) / 64);  // waves' worth of chains
+    double pass_us = D * (lds ? 0.01 + 0.0018 * units : 0.02 + 0.0075 * units);
+    if (D % 64 != 0)  // every output of the center sums scans all snapshots
+        pass_us += (lds ? 0.03 : 0.15) * N * (((int64_t)k * D + 1023) / 1024);
+    return 3.0 * pass_us >= (D > kIterC ? 7.4 : 3.7) * std::max(max_iters, 25);
+}
 
 extern "C" {
 
@@ -1100,14 +1121,7 @@ int ta_kmeans_ref(const float* snaps, int N, int D, int k, int max_iters, float*
                k);
     if (k > N) k = N;
     hipStream_t s = (hipStream_t)stream;
-    // one workgroup while its passes cost less than launches (about 10 us each
-    // that changes something, 2 us each after that, up to the cap): with the
-    // snapshots in its LDS (N D <= 32768) below k N D = 2^20 (64 x 512: k = 8
-    // 86 us against 102 with 25 passes launched, k = 32 127 against 96), read
-    // from global memory below 2^17 (32 x 1536, k = 2: 127 against 130; 96 x
-    // 512, k = 8: 373 against 99)
-    const bool small = (int64_t)k * N * D < (int64_t(1) << ((int64_t)N * D <= kXs ? 20 : 17));
-    if (!small && max_iters > 0 && max_iters <= kRefLaunches && k <= 65535) {
+    if (ref_launched(N, D, k, max_iters)) {
         KmeansScratch m;
         TA_REQUIRE(m.get(N, D, k, 0, s), "kmeans_ref: scratch allocation failed");
         tlaunch(k_kmeans_transpose, transpose_grid(N, D), dim3(256), s, snaps, m.xt, N,

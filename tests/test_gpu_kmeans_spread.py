@@ -48,12 +48,19 @@ def test_pp(N, D, k, iters, kind):
     assert np.allclose(host(M), rm, rtol=1e-12)
 
 
+# (the launches are taken by work per pass against the cap: all of these at 50,
+# none at 200; members past 4096 snapshots, a ragged last chunk of 64, more
+# centers than are resident at once)
+REF_LAUNCHED = [(64, 512, 64, 0), (300, 256, 12, 0), (130, 300, 40, 0), (1030, 33, 6, 0),
+                (4200, 64, 16, 0), (4229, 33, 16, 0), (20, 4100, 5, 0), (2050, 40, 2049, 0)]
+
+
 @pytest.mark.parametrize("kind", ["mixture", "spread", "dups"])
-@pytest.mark.parametrize("N,D,k,iters", SHAPES)
+@pytest.mark.parametrize("N,D,k,iters", SHAPES + REF_LAUNCHED)
 def test_ref(N, D, k, iters, kind):
     X, _ = data(N, D, kind)
     out = []
-    for cap in (50, 200):  # one launch per pass; the one-workgroup loop
+    for cap in (50, 200):  # one launch per pass (REF_LAUNCHED); the one-workgroup loop
         C = torch.empty(k * D, device=DEV)
         A = torch.empty(N, dtype=torch.int32, device=DEV)
         it = torch.empty(1, dtype=torch.int32, device=DEV)
@@ -64,38 +71,36 @@ def test_ref(N, D, k, iters, kind):
         assert np.array_equal(a, ra) and np.array_equal(c, rc) and i == ri
 
 
-def test_few_passes_match_the_loop():
-    """A cap below the passes the data needs: centers after the last update,
-    assignments of the last pass; no pass at all leaves the initial centers."""
-    X, _ = data(90, 64, "spread")
+@pytest.mark.parametrize("N,D,k", [(90, 64, 8), (300, 256, 12)])
+def test_few_passes_match_the_loop(N, D, k):
+    """A cap below the passes the data needs, in the one-workgroup loop and in
+    launches: centers after the last update, assignments of the last pass; no
+    pass at all leaves the initial centers."""
+    X, _ = data(N, D, "spread")
     for cap in (0, 1, 2, 3):
-        got = []
-        for big in (False, True):
-            C = torch.full((8 * 64,), -1.0, device=DEV)
-            A = torch.full((90,), -1, dtype=torch.int32, device=DEV)
-            it = torch.full((1,), -1, dtype=torch.int32, device=DEV)
-            call("ta_kmeans_ref", P(dev(X)), 90, 64, 8, cap, P(C), P(A), P(it), S())
-            got.append((host(C), host(A), host(it)))
-        want_c = X[[(i * 90) // 8 for i in range(8)]].copy()
-        asg, n_it = np.zeros(90, np.int32), 0
+        C = torch.full((k * D,), -1.0, device=DEV)
+        A = torch.full((N,), -1, dtype=torch.int32, device=DEV)
+        it = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+        call("ta_kmeans_ref", P(dev(X)), N, D, k, cap, P(C), P(A), P(it), S())
+        want_c = X[[(i * N) // k for i in range(k)]].copy()
+        asg, n_it = np.zeros(N, np.int32), 0
         for _ in range(cap):
-            d = np.zeros((90, 8), np.float32)
-            for i in range(64):
+            d = np.zeros((N, k), np.float32)
+            for i in range(D):
                 t = (X[:, None, i] - want_c[None, :, i]).astype(np.float32)
                 d = (d + (t * t).astype(np.float32)).astype(np.float32)
             a = d.argmin(1).astype(np.int32)
             if np.array_equal(a, asg):
                 break
             asg, n_it = a, n_it + 1
-            for c in range(8):
+            for c in range(k):
                 mem = np.nonzero(asg == c)[0]
-                s = np.zeros(64, np.float32)
+                s = np.zeros(D, np.float32)
                 for n in mem:
                     s = (s + X[n]).astype(np.float32)
                 want_c[c] = s / np.float32(len(mem)) if len(mem) else 0
-        for c, a, i in got:
-            assert np.array_equal(c.reshape(8, 64), want_c)
-            assert np.array_equal(a, asg) and int(i[0]) == n_it
+        assert np.array_equal(host(C).reshape(k, D), want_c)
+        assert np.array_equal(host(A), asg) and int(host(it)[0]) == n_it
 
 
 @pytest.mark.parametrize("pp", [True, False])
