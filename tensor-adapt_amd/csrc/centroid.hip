@@ -488,6 +488,95 @@ __global__ __launch_bounds__(1024) void k_kmeans_ref(const float* __restrict__ X
     if (threadIdx.x == 0 && iters_out) *iters_out = it;
 }
 
+// Stress-mode merge of a few short snapshots in one launch (the rule is at
+// ta_kmeans_pp): everything sits in LDS, and a pass costs its barriers and two
+// chains of D additions where a launch would cost more than that.  The same
+// chains in the same order as the launches below, so the same bits.  Passes
+// stop where one changes no assignment, as there.
+constexpr int kSmallX = 8192;        // N D and k D floats
+constexpr int kSmallN = 128;         // snapshots and centers
+constexpr int kSmallDist = 64 * 64;  // distances
+__global__ __launch_bounds__(1024) void k_kmeans_pp_small(const float* __restrict__ Xg,
+                                                          const float* __restrict__ W, int N, int D,
+                                                          int k, int iters, uint64_t seed,
+                                                          float* __restrict__ C_out,
+                                                          int32_t* __restrict__ asg_out,
+                                                          double* __restrict__ mass_out,
+                                                          int32_t* __restrict__ seeds_out) {
+    __shared__ __attribute__((aligned(16))) float X[kSmallX], C[kSmallX];
+    __shared__ float dist[kSmallDist], d2[kSmallN];
+    __shared__ int asg[kSmallN], chosen[kSmallN], order[kSmallN], rank_of[kSmallN];
+    __shared__ double mass[kSmallN];
+    const bool vec = D % 4 == 0;
+    for (int p = threadIdx.x; p < N * D; p += blockDim.x) X[p] = Xg[p];
+    uint64_t rng = seed;  // thread 0's
+    if (threadIdx.x == 0) {
+        const int first = (int)(u01(rng) * N);
+        chosen[0] = first >= N ? N - 1 : first;
+    }
+    if (threadIdx.x < N) {
+        d2[threadIdx.x] = FLT_MAX;
+        asg[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    for (int m = 1; m < k; m++) {
+        const int n[1] = {(int)threadIdx.x}, cm = chosen[m - 1];
+        if (n[0] < N) {
+            const float* const cb[1] = {X + cm * D};
+            const int kb[1] = {0};
+            float d[1];
+            sqdist_chains<1, 32>(X, D, 0, vec, n, cb, kb, d);
+            if (d[0] < d2[n[0]]) d2[n[0]] = d[0];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double total = 0.0, run = 0.0;
+            for (int i = 0; i < N; i++) total += (double)d2[i];
+            const double target = u01(rng) * total;
+            int pick = -1, last_pos = -1;
+            for (int i = 0; i < N; i++) {
+                run += (double)d2[i];
+                if (d2[i] > 0.f) last_pos = i;
+                if (pick < 0 && run > target && d2[i] > 0.f) pick = i;
+            }
+            chosen[m] = pick >= 0 ? pick : last_pos >= 0 ? last_pos : m % N;
+        }
+        __syncthreads();
+    }
+    for (int p = threadIdx.x; p < k * D; p += blockDim.x) C[p] = X[chosen[p / D] * D + p % D];
+    __syncthreads();
+    for (int it = 0; it <= iters; it++) {
+        const int changed = kmeans_assign(X, 0, vec, C, N, D, k, dist, asg);
+        if (it == iters || (it > 0 && !changed)) break;
+        kmeans_update(X, 0, C, N, D, k, asg, false);
+    }
+    // rank by member weight (F64, index order), stable descending
+    if (threadIdx.x == 0) {
+        for (int c = 0; c < k; c++) {
+            mass[c] = 0.0;
+            order[c] = c;
+        }
+        for (int n = 0; n < N; n++) mass[asg[n]] += (double)W[n];
+        for (int i = 1; i < k; i++) {
+            const int v = order[i];
+            int j = i - 1;
+            while (j >= 0 && mass[order[j]] < mass[v]) {
+                order[j + 1] = order[j];
+                j--;
+            }
+            order[j + 1] = v;
+        }
+        for (int r = 0; r < k; r++) rank_of[order[r]] = r;
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < k * D; p += blockDim.x) C_out[p] = C[order[p / D] * D + p % D];
+    if (threadIdx.x < N) asg_out[threadIdx.x] = rank_of[asg[threadIdx.x]];
+    if (threadIdx.x < k) {
+        if (mass_out) mass_out[threadIdx.x] = mass[order[threadIdx.x]];
+        if (seeds_out) seeds_out[threadIdx.x] = chosen[threadIdx.x];
+    }
+}
+
 // ── k-means spread over the GPU ───────────────────────────────────────────
 // Every value is a chain of F32 (or F64) additions that has to run in order,
 // so what the work costs is latency: the chains of a pass run side by side,
@@ -1161,8 +1250,23 @@ int ta_kmeans_pp(const float* snaps, const float* weights, int N, int D, int k, 
     if (k > N) k = N;
     TA_REQUIRE(k <= 1024, "kmeans_pp: k=%d exceeds 1024", k);
     hipStream_t s = (hipStream_t)stream;
+    // one workgroup where its draws (one at a time: 0.06 us per snapshot and
+    // 0.014 us per dimension, four times that where no 16-byte load fits, less
+    // the 0.6 us of a draw among the launches) cost less than the launches' fixed
+    // 13 us and what passes launched after the data has settled take, counted at
+    // 2 of their 3.7 us (fit to 2068 timed sizes, of which the slower form takes
+    // 1.41 times the other at worst; 4 x 16, k = 2: 7 us against 34 with 5 passes
+    // launched; 16 x 256, k = 4: 32 against 28 with one; 64 x 64, k = 64: 446
+    // against 115)
+    if (N <= kSmallN && (int64_t)N * D <= kSmallX && N * k <= kSmallDist &&
+        (int64_t)(k - 1) * (60 * N + 14 * (D % 4 ? 4 * D : D) - 600) <=
+            13000 + 2000 * ((int64_t)iters - 1)) {
+        tlaunch(k_kmeans_pp_small, dim3(1), dim3(1024), s, snaps, weights, N, D, k, iters, seed,
+                centers, assign, mass, seeds);
+        return check_launch("kmeans_pp");
+    }
     KmeansScratch m;
-    const bool pairs = N <= kPairMax;
+    const bool pairs = N <= kPairMax && k > 1;  // (one center: nothing is drawn by distance)
     TA_REQUIRE(m.get(N, D, k, pairs ? N : 1, s), "kmeans_pp: scratch allocation failed");
     tlaunch(k_kmeans_transpose, transpose_grid(N, D), dim3(256), s, snaps, m.xt, N, D);
     if (pairs)

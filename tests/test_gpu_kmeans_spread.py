@@ -30,10 +30,16 @@ def data(N, D, kind):
 
 SHAPES = [(1, 1, 1, 5), (2, 3, 2, 4), (63, 33, 9, 25), (64, 512, 32, 25), (65, 500, 32, 7),
           (130, 31, 40, 25), (1030, 17, 6, 12), (4200, 5, 4, 6), (20, 4100, 5, 6)]
+# the stress mode's one-workgroup form: its limits (128 snapshots, 8192 values,
+# 4096 distances) and one past each, both sides of its rule, passes that stop
+# early and none; centers past what is resident at once; one center
+PP_SMALL = [(1, 1, 1, 0), (4, 16, 2, 1000), (128, 64, 2, 25), (129, 63, 2, 25), (8, 1024, 2, 5),
+            (8, 1025, 2, 5), (64, 5, 64, 300), (65, 5, 64, 300), (16, 50, 8, 0), (16, 50, 8, 25),
+            (100, 12, 40, 200), (1100, 33, 1024, 4), (500, 70, 1, 3)]
 
 
 @pytest.mark.parametrize("kind", ["mixture", "spread", "dups"])
-@pytest.mark.parametrize("N,D,k,iters", SHAPES)
+@pytest.mark.parametrize("N,D,k,iters", SHAPES + PP_SMALL)
 def test_pp(N, D, k, iters, kind):
     X, W = data(N, D, kind)
     C = torch.empty(k * D, device=DEV)
