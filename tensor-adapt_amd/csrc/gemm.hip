@@ -2108,7 +2108,11 @@ struct SmallPlan {
     DeepPlan deep;
     int mid = 0;
 };
-static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split, bool capturing) {
+// capturing: called only where the answer matters (it is a runtime call: 0.5 us
+// of the 6.5 us a small product takes the host).
+template <typename Capturing>
+static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split,
+                            Capturing&& capturing) {
     SmallPlan p;
     p.mid = mid_bn(M, N, N > 3072 ? 256 : 192, ksteps, M >= 1024 && N >= 1024, 128);
     const bool big = p.mid == 0 && is_big_shape(M, N, ksteps);
@@ -2116,7 +2120,7 @@ static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split,
     // into the scratch pool, which may move before a replay)
     const bool fresh_split = M >= 128 && !big;
     p.deep = deep_plan(M, N, ksteps, may_split, 128);
-    if (p.deep.bn && p.deep.splits > 1 && fresh_split && capturing)
+    if (p.deep.bn && p.deep.splits > 1 && fresh_split && capturing())
         p.deep = deep_plan(M, N, ksteps, false, 128);
     if (p.deep.bn && big) {
         const int bn = big_bn(split256_variant(M, N, ksteps));
@@ -2241,8 +2245,9 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     if (xk && !yk && (K % BK) == 0 && vx && vy && N % 8 == 0 && N >= 64 && ldx < kMaxStageLd &&
         ldy < kMaxStageLd && auto_form && !lora_on) {
         // (as below: no scratch in a capture where the shape did not split)
-        const bool may_split = ksteps >= 16 || !is_capturing(s);
-        DeepPlan dp = deep_plan(M, N, ksteps, may_split, 128);
+        DeepPlan dp = deep_plan(M, N, ksteps, true, 128);
+        if (dp.splits > 1 && ksteps < 16 && is_capturing(s))
+            dp = deep_plan(M, N, ksteps, false, 128);
         if (!dp.bn) dp.bn = 128;
         a.tiles_m = (M + 127) / 128;
         a.tiles_n = (N + dp.bn - 1) / dp.bn;
@@ -2269,7 +2274,8 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     if (pipe_ok && (auto_form || g_big_variant == 19 || g_big_variant == 20)) {
         SmallPlan sp;
         if (auto_form)
-            sp = small_plan(M, N, ksteps, lora_on, force_splits != kUnsplit, is_capturing(s));
+            sp = small_plan(M, N, ksteps, lora_on, force_splits != kUnsplit,
+                            [s] { return is_capturing(s); });
         else
             sp.mid = g_big_variant == 19 ? 128 : 64;
         const DeepPlan& dp = sp.deep;
@@ -2957,7 +2963,8 @@ int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
         o[3] = p.deep.bn ? p.deep.splits : 1;
         return o[1] != TA_GEMM_TILES;
     };
-    if (small(N, small_plan(M, N, ks, lora != 0, true, captured != 0), out) ||
+    auto cap = [captured] { return captured != 0; };
+    if (small(N, small_plan(M, N, ks, lora != 0, true, cap), out) ||
         !is_big_shape(M, N, ks))
         return 0;
     const int variant = big_variant(M, N, ks, true), bn = big_bn(variant);
@@ -2968,7 +2975,7 @@ int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
     const int n_main = out[3] == 1 && variant == 18 ? tail_main_cols(M, N, ks) : 0;
     if (n_main) {
         out[0] = n_main;
-        small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, false, captured != 0), out + 4);
+        small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, false, cap), out + 4);
     }
     return 0;
 }
