@@ -2228,8 +2228,13 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     const bool big_shape = is_big_shape(M, N, ksteps);
     // K a LoRA rank (at most 64): k_gemm_rank.  The 128-row tiles below would
     // stage 64 k of zeros and write C two bytes at a time (8192 x 1536 x 16:
-    // 22 us, and 48 us with beta 1 and a K-strided Y)
-    if (xk && K <= 64 && N >= 64 && auto_form && !lora_on) {
+    // 22 us, and 48 us with beta 1 and a K-strided Y).  A whole 64-k stage of
+    // K-contiguous operands stays with the pipelined kernels, whose stores
+    // overlap other tiles (4096 x 3584 x 64: 11.5 us against 15.0), and up to 8
+    // rows whose C is read back with the tiles below (beta 1, 1 x 3584 x 48:
+    // 7.0 us against 8.2; 12 rows 8.6 against 8.1)
+    const bool few_rows = M <= 8 && K > 16 && beta != 0.f;
+    if (xk && K <= 64 && N >= 64 && auto_form && !lora_on && !pipe_ok && !few_rows) {
         a.tiles_m = (M + 63) / 64;
         a.tiles_n = (N + 255) / 256;
         const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n));

@@ -55,6 +55,10 @@ def test_small_gemm(M, N, K, beta, bias):
     # K of a rank: k_gemm_rank (odd ranks and strides load element by element)
     (1, 64, 2, 2, 0), (65, 257, 4, 4, 0), (64, 264, 16, 16, 0), (200, 896, 8, 24, 0),
     (129, 100, 33, 33, 3), (2331, 1536, 64, 64, 0),
+    # around its limits: up to 8 rows read back take the 32-wide tiles, a whole
+    # 64-k stage of K-contiguous operands the pipelined kernels
+    (8, 200, 48, 48, 0), (9, 200, 48, 48, 0), (8, 72, 16, 16, 0), (8, 18944, 64, 64, 0),
+    (130, 136, 64, 68, 4), (64, 8960, 64, 64, 0),
     # K-strided Y: one tile, ragged tiles, more waves of tiles, K splits
     (1, 64, 64, 64, 0), (130, 72, 128, 128, 8), (127, 200, 320, 320, 0), (64, 896, 4864, 4864, 0),
     (300, 1536, 1536, 1536, 16), (2100, 4872, 192, 192, 0),
