@@ -2111,7 +2111,7 @@ struct SmallPlan {
 // capturing: called only where the answer matters (it is a runtime call: 0.5 us
 // of the 6.5 us a small product takes the host).
 template <typename Capturing>
-static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split,
+static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool beta, bool may_split,
                             Capturing&& capturing) {
     SmallPlan p;
     p.mid = mid_bn(M, N, N > 3072 ? 256 : 192, ksteps, M >= 1024 && N >= 1024, 128);
@@ -2128,6 +2128,17 @@ static SmallPlan small_plan(int M, int N, int ksteps, bool lora, bool may_split,
         if (p.deep.us > 0.97 * split256_us(M, N, ksteps, t, split256_for(t, ksteps), lora))
             p.deep.bn = 0;
     }
+    // k_gemm_mid's two blocks per CU overlap one's epilogue with the other's
+    // products, which pays off where a 128-wide tile has few stages or reads C
+    // back (beta): 2048 x 2048 x 896 11.5 us against 13.7, x 1536 18.3 against
+    // 17.0; with beta x 256 8.2 against 9.5, x 1536 21.0 against 23.2, and with
+    // 152 tiles instead of 256 18.5 against 17.3.  64-wide tiles gain throughout.
+    if (p.mid && p.deep.bn == 128 && p.deep.splits == 1) {
+        const int64_t t = (int64_t)ceil_div(M, 128) * ceil_div(N, 128);
+        if (ksteps < 18 || (beta && (ksteps < 24 || t > 208))) p.deep.bn = 0;
+    }
+    // (up to 8 rows: the register-staged tiles; 1 x 18,944 x 64 7.2 us against 8.3)
+    if (!p.mid && p.deep.bn == 128 && beta && M <= 8 && ksteps <= 2) p.deep.bn = 0;
     return p;
 }
 
@@ -2279,7 +2290,7 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
     if (pipe_ok && (auto_form || g_big_variant == 19 || g_big_variant == 20)) {
         SmallPlan sp;
         if (auto_form)
-            sp = small_plan(M, N, ksteps, lora_on, force_splits != kUnsplit,
+            sp = small_plan(M, N, ksteps, lora_on, beta != 0.f, force_splits != kUnsplit,
                             [s] { return is_capturing(s); });
         else
             sp.mid = g_big_variant == 19 ? 128 : 64;
@@ -2956,7 +2967,7 @@ int ta_gemm_rm(int x_kmajor, int y_kmajor, int M, int N, int K, float alpha, con
                          ldc, bias, (hipStream_t)stream, 0, nullptr);
 }
 
-int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
+int ta_gemm_plan(int M, int N, int K, int lora, int beta, int captured, int32_t* out) {
     TA_REQUIRE(M > 0 && N > 0 && K > 0 && K % BK == 0 && out,
                "gemm_plan: M, N, K > 0 and K a multiple of %d", BK);
     const int ks = K / BK;
@@ -2969,7 +2980,7 @@ int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
         return o[1] != TA_GEMM_TILES;
     };
     auto cap = [captured] { return captured != 0; };
-    if (small(N, small_plan(M, N, ks, lora != 0, true, cap), out) ||
+    if (small(N, small_plan(M, N, ks, lora != 0, beta != 0, true, cap), out) ||
         !is_big_shape(M, N, ks))
         return 0;
     const int variant = big_variant(M, N, ks, true), bn = big_bn(variant);
@@ -2980,7 +2991,7 @@ int ta_gemm_plan(int M, int N, int K, int lora, int captured, int32_t* out) {
     const int n_main = out[3] == 1 && variant == 18 ? tail_main_cols(M, N, ks) : 0;
     if (n_main) {
         out[0] = n_main;
-        small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, false, cap), out + 4);
+        small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, beta != 0, false, cap), out + 4);
     }
     return 0;
 }

@@ -15,9 +15,9 @@ import tadapt
 TILES, DEEP, MID, BIG = range(4)
 
 
-def plan(M, N, K, lora=1, captured=0):
+def plan(M, N, K, lora=1, beta=0, captured=0):
     out = (ctypes.c_int32 * 8)()
-    tadapt.call("ta_gemm_plan", M, N, K, lora, captured, ctypes.addressof(out))
+    tadapt.call("ta_gemm_plan", M, N, K, lora, beta, captured, ctypes.addressof(out))
     rows = [tuple(out[:4]), tuple(out[4:])]
     return [r for r in rows if r[0]]
 
@@ -55,3 +55,16 @@ def test_tail_of_a_wide_intermediate():
     tiles, of which the last 128 columns run apart."""
     rows = plan(2048, 8320, 1536)
     assert len(rows) == 2 and rows[1] == (128, DEEP, 64, 1), rows
+
+
+def test_short_k_runs_two_blocks_per_cu():
+    """Where both were timed, the 128-row forms' choice: 128-wide tiles of few
+    stages, or with C read back, run k_gemm_mid's two blocks per CU."""
+    for M, N in ((2048, 2048), (8192, 512), (1024, 3584)):
+        for K in (64, 256, 512, 896, 1024):
+            assert plan(M, N, K, 0)[0][1] == MID, (M, N, K)
+            assert plan(M, N, K, 0, beta=1)[0][1] == MID, (M, N, K)
+        assert plan(M, N, 1536, 0)[0][1:4] == (DEEP, 128, 1)
+        assert plan(M, N, 1536, 0, beta=1)[0][1] == MID
+    assert plan(512, 4864, 1536, 0, beta=1)[0][1:4] == (DEEP, 128, 1)
+    assert plan(2048, 896, 896, 0, beta=1)[0][1:4] == (DEEP, 64, 1)
