@@ -2033,15 +2033,19 @@ static double split_us(int M, int N, int splits, double gbs) {
 // choice within 1.5% of the best measured one): a fixed 4.3 us (64-wide) or
 // 5 us (128-wide), and per 64-k stage 0.27 or 0.36 us on an empty chip, 45%
 // more with all 256 CUs loading; 2 us and 4 TB/s for the partials of a
-// split.  So K = 896 .. 1536 runs unsplit, and a long K over few tiles
-// splits until the partials cost what the stages gain (128 x 896 x 4864:
-// 23.2 us unsplit, 16.1, 11.9, 10.6 and 12.2 us in 2, 4, 8 and 16 splits).
+// split.  A split is two launches, which take 10 us however little they do
+// (128 x 256 x 1024: 10.0 us in two splits, 8.5 unsplit), so it is taken only
+// where the unsplit form takes longer than that: a few tiles over K = 1536
+// (128 x 896: 11.1 unsplit, 10.1 in four), a long K until the partials cost
+// what the stages gain (128 x 896 x 4864: 23.2 us unsplit, 16.1, 11.9, 10.6
+// and 12.2 us in 2, 4, 8 and 16 splits).
 struct DeepPlan {
     int bn = 0, splits = 1;
     double us = 1e30;
 };
+constexpr double kSplitLeastUs = 10.0;
 static DeepPlan deep_plan(int M, int N, int ksteps, bool can_split, int n_mult) {
-    DeepPlan best;
+    DeepPlan best, split;
     if (N < 64) return best;
     for (int bn = 64; bn <= 128; bn *= 2) {
         if (n_mult % bn != 0) continue;
@@ -2054,15 +2058,16 @@ static DeepPlan deep_plan(int M, int N, int ksteps, bool can_split, int n_mult) 
             const double load = 1.0 + 0.45 * (double)t * sp / 256.0;
             const double us = (bn == 64 ? 4.3 + 0.27 * load * per : 5.0 + 0.36 * load * per) +
                               split_us(M, N, sp, 4000.0);
-            if (us < best.us) {
-                best.bn = bn;
-                best.splits = sp;
-                best.us = us;
+            DeepPlan& b = sp > 1 ? split : best;
+            if (us < b.us) {
+                b.bn = bn;
+                b.splits = sp;
+                b.us = us;
             }
             if (q >= most) break;
         }
     }
-    return best;
+    return split.us < best.us && kSplitLeastUs < best.us ? split : best;
 }
 // Expected time of the 256-row kernels on a long-K product (ksteps >= 32) of
 // `tiles` tiles in `splits` splits: 7 us and 1.35 us per 64-k stage for each

@@ -68,3 +68,11 @@ def test_short_k_runs_two_blocks_per_cu():
         assert plan(M, N, 1536, 0, beta=1)[0][1] == MID
     assert plan(512, 4864, 1536, 0, beta=1)[0][1:4] == (DEEP, 128, 1)
     assert plan(2048, 896, 896, 0, beta=1)[0][1:4] == (DEEP, 64, 1)
+
+
+def test_splits_pay_for_their_second_launch():
+    """Two launches take 10 us, so K = 1024 over a few tiles runs unsplit."""
+    for M, N in ((128, 128), (128, 256), (256, 128)):
+        assert plan(M, N, 1024, 0)[0][1:4] == (DEEP, 64, 1)
+    assert plan(128, 896, 1536, 0)[0][1:4] == (DEEP, 64, 4)
+    assert plan(128, 896, 4864, 0)[0][3] > 4
