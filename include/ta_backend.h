@@ -194,10 +194,12 @@ int ta_gemm_rm_variant(int variant, int x_kmajor, int y_kmajor, int M, int N, in
 
 /* How ta_gemm_rm (and the step engine) runs a K-contiguous product of 16-byte
  * aligned operands, K a multiple of 64: out holds one or two launches of
- * {columns, form, tile width, K splits}, the second (columns 0 when there is
- * none) the columns past the last whole wave of 256 x 256 tiles.  lora: rank-r
- * terms follow; beta: C is read back; captured: the stream records a graph.
- * Host arithmetic only.  No reference counterpart. */
+ * {columns, form, tile width, K splits, tiles in launch order}, the second
+ * (columns 0 when there is none) the columns past the last whole wave of 256 x
+ * 256 tiles.  lora: rank-r terms follow; beta: C is read back; captured: the
+ * stream records a graph, where products of 128 or more rows that only the
+ * small-output form splits run unsplit (another order of the same sums, so not
+ * always the eager bits).  Host arithmetic only.  No reference counterpart. */
 enum { TA_GEMM_TILES = 0, TA_GEMM_DEEP = 1, TA_GEMM_MID = 2, TA_GEMM_BIG = 3 };
 int ta_gemm_plan(int M, int N, int K, int lora, int beta, int captured, int32_t* out);
 

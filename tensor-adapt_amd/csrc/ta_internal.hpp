@@ -101,10 +101,12 @@ __device__ __forceinline__ float sum_splits(const float* __restrict__ part, int 
 // split-K grid an XCD so works few splits and reads a fraction of K of both
 // operands, where one range of tiles for every split would have each XCD
 // read all of K.
-__device__ __forceinline__ int xcd_band() {
-    const int total = gridDim.x * gridDim.z, lin = blockIdx.z * gridDim.x + blockIdx.x;
+__device__ __forceinline__ int xcd_band_of(int total, int lin) {
     const int q = total >> 3, r = total & 7, x = lin & 7;
     return x * q + min(x, r) + (lin >> 3);
+}
+__device__ __forceinline__ int xcd_band() {
+    return xcd_band_of(gridDim.x * gridDim.z, blockIdx.z * gridDim.x + blockIdx.x);
 }
 
 // LoRA terms for gemm_dispatch.  After the base epilogue, for each pair p

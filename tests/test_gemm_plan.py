@@ -16,9 +16,9 @@ TILES, DEEP, MID, BIG = range(4)
 
 
 def plan(M, N, K, lora=1, beta=0, captured=0):
-    out = (ctypes.c_int32 * 8)()
+    out = (ctypes.c_int32 * 10)()
     tadapt.call("ta_gemm_plan", M, N, K, lora, beta, captured, ctypes.addressof(out))
-    rows = [tuple(out[:4]), tuple(out[4:])]
+    rows = [tuple(out[:5]), tuple(out[5:])]
     return [r for r in rows if r[0]]
 
 
@@ -54,7 +54,7 @@ def test_tail_of_a_wide_intermediate():
     """2048 tokens, hidden 1536, intermediate 8320, down_proj adapted: 264
     tiles, of which the last 128 columns run apart."""
     rows = plan(2048, 8320, 1536)
-    assert len(rows) == 2 and rows[1] == (128, DEEP, 64, 1), rows
+    assert len(rows) == 2 and rows[1] == (128, DEEP, 64, 1, 0), rows
 
 
 def test_short_k_runs_two_blocks_per_cu():
@@ -76,3 +76,12 @@ def test_splits_pay_for_their_second_launch():
         assert plan(M, N, 1024, 0)[0][1:4] == (DEEP, 64, 1)
     assert plan(128, 896, 1536, 0)[0][1:4] == (DEEP, 64, 4)
     assert plan(128, 896, 4864, 0)[0][3] > 4
+
+
+@pytest.mark.parametrize("M,N,K,order", [
+    (4864, 3584, 18944, 1), (5888, 3584, 18944, 1), (9472, 3584, 12288, 1), (16640, 1536, 1536, 1),
+    (4864, 18944, 3584, 0), (2331, 151936, 1536, 0), (3328, 8960, 1536, 0), (4864, 3584, 8192, 0),
+    (3840, 3584, 18944, 0), (8192, 3584, 18944, 0)])
+def test_launch_order(M, N, K, order):
+    """The products that ran slower with each XCD on a range of tiles of its own."""
+    assert plan(M, N, K, 0)[0][4] == order
