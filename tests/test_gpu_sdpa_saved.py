@@ -1,7 +1,7 @@
 """The attention with stored probabilities at the edges of its 64-row tiles,
 with rows that start on and off a 16-byte boundary (T a multiple of 4 or
-not), and with an infinite value at a key, which must not reach the rows
-before it.  P against F64 to F32 accuracy; O, dQ, dK and dV to one BF16
+not), and with an infinite value at a key, which must not reach the query
+tiles before it.  P against F64 to F32 accuracy; O, dQ, dK and dV to one BF16
 rounding of sums whose P or dS factors keep 16 bits (relative L2 4e-3)."""
 import math
 
@@ -55,11 +55,11 @@ def test_saved_probabilities(T, hd):
 
 
 def test_infinite_value_stays_behind_the_mask():
-    """Rows before an infinite V row see neither it nor a NaN from it, in D
-    (dK of keys the infinite row does not attend from) or in O."""
+    """Query tiles before an infinite V row see neither it nor a NaN from it in
+    O and dQ; P and dV take nothing from V."""
     B, T, Hq, Hk, hd = 1, 190, 2, 1, 64
     q, k, v, do = inputs(B, T, Hq, Hk, hd)
     v[150] = float("inf")
     o, p, dq, dk, dv = run(B, T, Hq, Hk, hd, q, k, v, do)
     assert bool(torch.isfinite(o[:128]).all()) and bool(torch.isfinite(p).all())
-    assert bool(torch.isfinite(dv).all())
+    assert bool(torch.isfinite(dv).all()) and bool(torch.isfinite(dq[:128]).all())
