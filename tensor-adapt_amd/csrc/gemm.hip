@@ -2054,17 +2054,18 @@ static double split_us(int M, int N, int splits, double gbs) {
 
 // Tile width and K splits of k_gemm_deep for an M x N x K product (bn 0: not
 // this kernel), with the time it is expected to take.  The kernel runs one
-// block per CU, so only grids of at most 256 blocks qualify.  The model,
-// fitted to 290 measured (shape, width, splits) times (geometric mean of the
-// choice within 1.5% of the best measured one): a fixed 4.3 us (64-wide) or
-// 5 us (128-wide), and per 64-k stage 0.27 or 0.36 us on an empty chip, 45%
-// more with all 256 CUs loading; 2 us and 4 TB/s for the partials of a
-// split.  A split is two launches, which take 10 us however little they do
-// (128 x 256 x 1024: 10.0 us in two splits, 8.5 unsplit), so it is taken only
-// where the unsplit form takes longer than that: a few tiles over K = 1536
-// (128 x 896: 11.1 unsplit, 10.1 in four), a long K until the partials cost
-// what the stages gain (128 x 896 x 4864: 23.2 us unsplit, 16.1, 11.9, 10.6
-// and 12.2 us in 2, 4, 8 and 16 splits).
+// block per CU, so only grids of at most 256 blocks qualify.  The model: a
+// fixed 4.3 us (64-wide) or 5 us (128-wide), and per 64-k stage 0.27 or 0.36
+// us on an empty chip, 45% more with all 256 CUs loading; 2 us and 4 TB/s for
+// the partials of a split.  Its choices are within 0.5% of the best of 685
+// times of 135 products in the geometric mean, 15% at worst (256 x 1536 x 1536:
+// 14.0 us unsplit, 12.2 in four splits).  A split is two launches, which take
+// the host alone about 10 us a call (128 x 256 x 1024 call after call: 10.0 us
+// in two splits, 8.5 unsplit), so it is taken only where the unsplit form takes
+// longer than that: a few tiles over K = 1536 (128 x 896: 11.1 unsplit, 10.1 in
+// four), a long K until the partials cost what the stages gain (128 x 896 x
+// 4864: 23.2 us unsplit, 16.1, 11.9, 10.6 and 12.2 us in 2, 4, 8 and 16
+// splits).
 struct DeepPlan {
     int bn = 0, splits = 1;
     double us = 1e30;
