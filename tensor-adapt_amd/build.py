@@ -19,7 +19,7 @@ BUILD = os.path.join(CSRC, "_build")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-# -packed-fp32-ops off: packed F32 VALU forms are avoided on this pool.
+# -packed-fp32-ops off: some packed F32 VALU forms have given wrong results.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall",
          "-Wno-unused-function", "-Wno-unused-variable",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

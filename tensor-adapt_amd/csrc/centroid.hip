@@ -583,7 +583,7 @@ __global__ __launch_bounds__(1024) void k_kmeans_pp_small(const float* __restric
 // one per lane, and a Lloyd iteration is one launch of one block per center
 // (k_kmeans_iter) with nothing to wait for inside a launch.  The snapshots
 // are kept transposed as well, so that 64 chains read 64 neighbouring values.
-// 64 snapshots of 512, k = 32, 25 passes: 139 us, against 844 us with the
+// 64 snapshots of 512, k = 32, 25 passes: 126 us, against 849 us with the
 // distances spread out and everything else on one workgroup, and 3.1 ms on
 // one workgroup alone.
 
@@ -830,9 +830,10 @@ __device__ __forceinline__ int nearest64(const float* __restrict__ dist, int N, 
 }
 
 // Iteration `it` of Lloyd's loop, block c for center c: every snapshot's
-// nearest center from the distances din [k][N] (each block for itself: N x k
-// loads), center c as the mean of its members summed in snapshot index order,
-// and the new center's distances into dout.  An empty center becomes zero
+// nearest center from the distances din [k][N], center c as the mean of its
+// members summed in snapshot index order, and the new center's distances into
+// dout.  Each block forms the assignments for itself, k^2 N cached loads a pass:
+// 2.6 ms a pass at 4096 x 64 into 1024, against 38 ms on one workgroup.  An empty center becomes zero
 // (REF, the reference's loop) or stays.  A pass that changes no assignment
 // ends the loop: the centers and distances of every later pass would be the
 // same values, so *done makes later launches return at once.

@@ -45,7 +45,7 @@ struct Scratch {
     size_t bytes = 0;
 };
 static std::mutex g_scratch_mu;
-constexpr int kSlots = 4;  // 0: reduction partials, 1: operand staging, 2-3: spare
+constexpr int kSlots = 4;  // 0: partials of splits and reductions, 2: attention dK/dV partials; 1, 3: spare
 struct ScratchSet {
     Scratch slot[kSlots];
 };
