@@ -65,7 +65,6 @@ struct GemmArgs {
     float* part;     // split-K partials [splits][M][N]
     int k_per_split; // multiple of BK
     int tiles_m, tiles_n;
-    int launch_order;  // unsplit grids: blocks take the tiles in launch order
     // LoRA epilogue (k_gemm_big only): after the base rounding, for each
     // pair p in order, with D_p = U_p V_p^T (U_p [M x r], V_p [N x r]):
     //   delta: C = bf16(C + s * bf16(D_p))    (apply_lora_fwd)
@@ -294,16 +293,35 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a, bool vecx, bool vecy) 
 // ── Large K-contiguous GEMMs (every frozen-base projection, the LM head) ──
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Whether an unsplit grid of `tiles` tiles over N columns (rounded up to whole
+// tiles) takes them in launch order: blocks go round-robin over the XCDs, so
+// all of them then work the same few bands.
+// With more than one wave of tiles, more rows than columns and operands past
+// the 256 MB of last-level cache, the XCDs' separate ranges of rows push each
+// other's bands out (4864 x 3584 x 18944: 786 us in ranges, 721 in launch
+// order; 5888 x 3584 873, 772; 9472 x 3584 x 12288 802, 747); with few columns
+// they gain nothing to begin with (16,640 x 1536 x 1536 87, 86).  Elsewhere
+// ranges are as fast or faster (2331 x 151,936 x 1536 1057 us, 1122 in launch
+// order; 4864 x 18,944 x 3584 511, 547; 3328 x 8960 x 1536 82, 87).  A multiple
+// of 8 tiles runs in ranges of equal length and was not timed the other way.
+// (Formed in the kernel from what it has loaded anyway: a flag among the
+// arguments made the SwiGLU form 3% slower in their midst and short launches
+// 0.1-0.3 us slower at their end.)
+constexpr bool tile_launch_order(int64_t M, int64_t N, int64_t K, int tiles) {
+    return tiles > 256 && (tiles & 7) != 0 && M > N &&
+           (N <= 1536 || 2 * K * (M + N) > (int64_t(256) << 20));
+}
+
 // Tile of a block for the large kernels.  Blocks are dealt round-robin to
 // the 8 XCDs (each with its own L2); each XCD gets a contiguous range of
 // tile indices, walked in groups of GM tile-rows column by column, so the
 // ~32 tiles an XCD runs at once share GM row bands of X and a few column
 // bands of Y in its L2 instead of streaming all of Y.  GM = 8 (8 x 4
 // tiles at once) measured 0.4% faster on the c3 step than 4 (4 x 8) and
-// 1% faster than 16.  launch_order: the tiles go in block order instead
-// (tile_launch_order).
+// 1% faster than 16.  BN: the tile width of grids that tile_launch_order may
+// put in launch order (0: always ranges).
 constexpr int TILE_GM = 8;
-template <bool SPLIT>
+template <bool SPLIT, int BN>
 __device__ __forceinline__ void big_tile(const GemmArgs& a, int& tm, int& tn, int& zs) {
     const int nt = a.tiles_m * a.tiles_n;
     int bid;
@@ -315,7 +333,9 @@ __device__ __forceinline__ void big_tile(const GemmArgs& a, int& tm, int& tn, in
     } else {
         // (an unsplit grid is the tiles: no load of the grid's size, 0.2 us of a
         // tile's start)
-        bid = a.launch_order ? (int)blockIdx.x : xcd_band_of(nt, blockIdx.x);
+        bid = BN > 0 && tile_launch_order(a.M, a.tiles_n * BN, a.K, nt)
+                  ? (int)blockIdx.x
+                  : xcd_band_of(nt, blockIdx.x);
     }
     int gsz = TILE_GM * a.tiles_n;
     int g = bid / gsz, idx = bid % gsz;
@@ -708,7 +728,7 @@ __global__ __launch_bounds__(WMW * WNW * 64) void k_gemm_dma(GemmArgs a) {
 
     int tm_i, tn_i;
     int zs;
-    big_tile<EPI == EPI_PARTIAL>(a, tm_i, tn_i, zs);
+    big_tile<EPI == EPI_PARTIAL, 0>(a, tm_i, tn_i, zs);
     int m0 = tm_i * BM, n0 = tn_i * BN;
     int kbeg = zs * a.k_per_split;
     if constexpr (EPI == EPI_PARTIAL) a.part += (int64_t)zs * a.M * a.N;
@@ -1216,7 +1236,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pipe_body(const GemmA
 
     int tm_i, tn_i;
     int zs;  // split (PART)
-    big_tile<PART>(a0, tm_i, tn_i, zs);
+    big_tile<PART, SWIGLU ? 0 : BN>(a0, tm_i, tn_i, zs);
     // N-concatenated groups: this tile's group supplies Y, C, N, bias, LoRA
     GemmArgs a = a0;
     if (a0.ngroups > 1) {
@@ -2031,21 +2051,6 @@ static bool is_capturing(hipStream_t s) {
 }
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// Whether an unsplit grid of `tiles` tiles takes them in launch order: blocks
-// go round-robin over the XCDs, so all of them then work the same few bands.
-// With more than one wave of tiles, more rows than columns and operands past
-// the 256 MB of last-level cache, the XCDs' separate ranges of rows push each
-// other's bands out (4864 x 3584 x 18944: 786 us in ranges, 721 in launch
-// order; 5888 x 3584 873, 772; 9472 x 3584 x 12288 802, 747); with few columns
-// they gain nothing to begin with (16,640 x 1536 x 1536 87, 86).  Elsewhere
-// ranges are as fast or faster (2331 x 151,936 x 1536 1057 us, 1122 in launch
-// order; 4864 x 18,944 x 3584 511, 547; 3328 x 8960 x 1536 82, 87).  A multiple
-// of 8 tiles runs in ranges of equal length and was not timed the other way.
-static bool tile_launch_order(int64_t M, int64_t N, int64_t K, int64_t tiles) {
-    return tiles > 256 && tiles % 8 != 0 && M > N &&
-           (N <= 1536 || 2 * K * (M + N) > (int64_t(256) << 20));
-}
-
 // F32 partials of an M x N output written and read back over `splits`: the
 // reduce's launch and the traffic at the rate it measured (GB/s).
 static double split_us(int M, int N, int splits, double gbs) {
@@ -2366,7 +2371,6 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
             a.tiles_m = (M + 127) / 128;
             a.tiles_n = (N + bn - 1) / bn;
             a.k_per_split = K;
-            a.launch_order = tile_launch_order(M, N, K, (int64_t)a.tiles_m * a.tiles_n);
             set_lora();
             const bool timed = kprof_begin(KP_GEMM_BIG, s);
             dim3 grid(a.tiles_m * a.tiles_n);
@@ -2453,7 +2457,6 @@ int gemm_dispatch(bool xk, bool yk, int M, int N, int K, float alpha, const bf16
         const bool fuse = lora && lora->n > 0 && (lora->r & 7) == 0 &&
                           (!is_pipe(variant) || lora->r <= 64);
         if (fuse) set_lora();
-        a.launch_order = tile_launch_order(M, N, K, tiles);
         // measurement hook: algorithmic work of the launch (MNK product,
         // rank-r epilogue products; operands read once, C written once and
         // read once more when beta != 0)
@@ -2642,7 +2645,6 @@ int gemm_chain(int M, int N, const GemmSeg* sg, int ns, bf16* C, int64_t ldc, co
     const int bn = deep ? deep : mid ? mid : BNb;
     a.tiles_m = deep || mid ? (M + 127) / 128 : (M + 255) / 256;
     a.tiles_n = (N + bn - 1) / bn;
-    a.launch_order = tile_launch_order(M, N, Ktot, (int64_t)a.tiles_m * a.tiles_n);
     a.ngroups = 1;
     a.nseg = ns;
     int k = 0;
@@ -2797,7 +2799,6 @@ int gemm_groups(int M, int K, const bf16* X, int64_t ldx, int64_t ldy, const Gem
     a.k_per_split = K;
     a.tiles_m = deep || mid ? (M + 127) / 128 : (M + 255) / 256;
     a.tiles_n = Ntot / TBN;
-    a.launch_order = tile_launch_order(M, Ntot, K, (int64_t)a.tiles_m * a.tiles_n);
     a.ngroups = ng;
     a.lora_r = l0 ? l0->r : 0;
     a.lora_delta = l0 && l0->delta ? 1 : 0;
@@ -3014,7 +3015,8 @@ int ta_gemm_plan(int M, int N, int K, int lora, int beta, int captured, int32_t*
         o[2] = p.deep.bn ? p.deep.bn : p.mid;
         o[3] = p.deep.bn ? p.deep.splits : 1;
         if (o[1] == TA_GEMM_MID)
-            o[4] = tile_launch_order(M, n, K, (int64_t)ceil_div(M, 128) * ceil_div(n, p.mid));
+            o[4] = tile_launch_order(M, ceil_div(n, p.mid) * p.mid, K,
+                                     ceil_div(M, 128) * ceil_div(n, p.mid));
         return o[1] != TA_GEMM_TILES;
     };
     auto cap = [captured] { return captured != 0; };
@@ -3031,7 +3033,8 @@ int ta_gemm_plan(int M, int N, int K, int lora, int beta, int captured, int32_t*
         out[0] = n_main;
         small(N - n_main, small_plan(M, N - n_main, ks, lora != 0, beta != 0, false, cap), out + 5);
     }
-    out[4] = out[3] == 1 && tile_launch_order(M, out[0], K, (int64_t)ceil_div(M, 256) * ceil_div(out[0], bn));
+    const int tn = ceil_div(out[0], bn);
+    out[4] = out[3] == 1 && tile_launch_order(M, tn * bn, K, ceil_div(M, 256) * tn);
     return 0;
 }
 
